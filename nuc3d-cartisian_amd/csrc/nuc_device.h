@@ -37,20 +37,28 @@ __device__ __forceinline__ T w7_sos(T a, T b, T c, T d, bool outer)
     return k0 * e0 * e0 + k1 * e1 * e1 + T(203060.0 / 1063.0) * g2 * g2;
 }
 
-// 7-point WENO with Z weights, src/weno7js.cpp:79-133 (eps 1e-20); hccs
-// closures use the same formula with eps 1e-40 (src/hccs.cpp:85-135), hccs78
-// edges with 1e-20 (src/hccs78.cpp:246-304).
+// reciprocal: hardware estimate refined by two Newton steps (|err| <= 1 ulp)
+__device__ __forceinline__ double frcp(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    double e = fma(-x, r, 1.0);
+    r = fma(r, e, r);
+    e = fma(-x, r, 1.0);
+    return fma(r, e, r);
+}
+// FP32 (mixed path): the hardware reciprocal, 1 ulp
+__device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
+
+// 7-point WENO stencil, src/weno7js.cpp:79-118: smoothness indicators b and
+// candidate values q of f[0..6].
 // FP64 stencils: the smoothness indicators are the reference's expanded
 // quadratic forms, whose coefficients (up to 17246) cancel to O(h^2) on smooth
 // data, so any reassociation or FMA moves them by ~1e-6 relative and shifts
 // the Z weights.  They are therefore evaluated without contraction and in the
 // reference's operation order, which makes them bit-identical to the
 // reference.  FP32 stencils (the mixed path) use the sums of squares above.
-// T: indicators and candidate values; TW: the nonlinear weights (the Z
-// weights square tau/(eps+is) with eps 1e-20/1e-40, outside FP32's range).
-// asum receives the sum of the unnormalised weights (hccs78's blend factor).
-template <typename T, typename TW>
-__device__ __forceinline__ TW weno7z(const T *f, TW eps, TW &asum)
+template <typename T>
+__device__ __forceinline__ void weno7_stencil(const T *f, T b[4], T q[4])
 {
 #pragma clang fp contract(off)
     T is0, is1, is2, is3;
@@ -73,59 +81,80 @@ __device__ __forceinline__ TW weno7z(const T *f, TW eps, TW &asum)
             + f[4] * (T(11003) * f[4] - T(17246) * f[5] + T(4642) * f[6])
             + f[5] * (T(7043) * f[5] - T(3882) * f[6]) + T(547) * f[6] * f[6];
     }
-    T q0 = T(-3.0 / 12.0) * f[0] + T(13.0 / 12.0) * f[1] + T(-23.0 / 12.0) * f[2] + T(25.0 / 12.0) * f[3];
-    T q1 = T(1.0 / 12.0) * f[1] + T(-5.0 / 12.0) * f[2] + T(13.0 / 12.0) * f[3] + T(3.0 / 12.0) * f[4];
-    T q2 = T(-1.0 / 12.0) * f[2] + T(7.0 / 12.0) * f[3] + T(7.0 / 12.0) * f[4] + T(-1.0 / 12.0) * f[5];
-    T q3 = T(3.0 / 12.0) * f[3] + T(13.0 / 12.0) * f[4] + T(-5.0 / 12.0) * f[5] + T(1.0 / 12.0) * f[6];
-    const TW b0 = is0, b1 = is1, b2 = is2, b3 = is3;
-    TW tau = fabs(b0 - b3);
-    TW a0 = TW(1.0 / 35.0) * (TW(1) + sq(tau / (eps + b0)));
-    TW a1 = TW(12.0 / 35.0) * (TW(1) + sq(tau / (eps + b1)));
-    TW a2 = TW(18.0 / 35.0) * (TW(1) + sq(tau / (eps + b2)));
-    TW a3 = TW(4.0 / 35.0) * (TW(1) + sq(tau / (eps + b3)));
-    asum = a0 + a1 + a2 + a3;
-    return a0 / asum * TW(q0) + a1 / asum * TW(q1) + a2 / asum * TW(q2) + a3 / asum * TW(q3);
+    q[0] = T(-3.0 / 12.0) * f[0] + T(13.0 / 12.0) * f[1] + T(-23.0 / 12.0) * f[2] + T(25.0 / 12.0) * f[3];
+    q[1] = T(1.0 / 12.0) * f[1] + T(-5.0 / 12.0) * f[2] + T(13.0 / 12.0) * f[3] + T(3.0 / 12.0) * f[4];
+    q[2] = T(-1.0 / 12.0) * f[2] + T(7.0 / 12.0) * f[3] + T(7.0 / 12.0) * f[4] + T(-1.0 / 12.0) * f[5];
+    q[3] = T(3.0 / 12.0) * f[3] + T(13.0 / 12.0) * f[4] + T(-5.0 / 12.0) * f[5] + T(1.0 / 12.0) * f[6];
+    b[0] = is0; b[1] = is1; b[2] = is2; b[3] = is3;
+}
+
+// The Z-weighted value of that stencil (eps 1e-20: src/weno7js.cpp:119-133,
+// src/hccs78.cpp:246-304; 1e-40: the hccs closures, src/hccs.cpp:85-135).
+// T: indicators and candidate values; TW: the nonlinear weights (they square
+// tau/(eps+is) with eps 1e-20/1e-40, outside FP32's range).
+// X receives the sum of the unnormalised weights less 1, sum c_k t_k^2 with
+// t_k = tau/(eps+is_k), formed without the cancellation of that difference;
+// the hccs family blends by theta = 1/(1 + X^2).
+// Bound by FP64 issue: the eight IEEE quotients of the plain form are about
+// 90 of a row's 210 instructions.  Here the four t_k share two reciprocals
+// (of is_0 is_1 and is_2 is_3, whose products stay in range: eps^2 >= 1e-80)
+// and the normalisation is one.  Errors over random and smooth indicators
+// against 80-bit: 1.3e-16 rms in both forms.
+template <typename T, typename TW>
+__device__ __forceinline__ TW weno7z(const T *f, TW eps, TW &X)
+{
+    T is[4], q[4];
+    weno7_stencil<T>(f, is, q);
+    const TW s0 = eps + TW(is[0]), s1 = eps + TW(is[1]), s2 = eps + TW(is[2]), s3 = eps + TW(is[3]);
+    const TW tau = fabs(TW(is[0]) - TW(is[3]));
+    const TW r01 = tau * frcp(s0 * s1), r23 = tau * frcp(s2 * s3);
+    const TW x0 = TW(1.0 / 35.0) * sq(r01 * s1), x1 = TW(12.0 / 35.0) * sq(r01 * s0);
+    const TW x2 = TW(18.0 / 35.0) * sq(r23 * s3), x3 = TW(4.0 / 35.0) * sq(r23 * s2);
+    X = (x0 + x1) + (x2 + x3);
+    const TW a0 = TW(1.0 / 35.0) + x0, a1 = TW(12.0 / 35.0) + x1;
+    const TW a2 = TW(18.0 / 35.0) + x2, a3 = TW(4.0 / 35.0) + x3;
+    return (a0 * TW(q[0]) + a1 * TW(q[1]) + a2 * TW(q[2]) + a3 * TW(q[3])) * frcp((a0 + a1) + (a2 + a3));
 }
 
 template <typename T, typename TW>
 __device__ __forceinline__ TW weno7z(const T *f, TW eps)
 {
-    TW asum;
-    return weno7z<T, TW>(f, eps, asum);
+    TW X;
+    return weno7z<T, TW>(f, eps, X);
 }
 
-// hccs78 inner point, src/hccs78.cpp:66-117: the WENO7-Z value (eps 1e-20)
-// blended with the 8-point central value through theta = 1/(1 + (asum-1)^2).
+// hccs78, src/hccs78.cpp:66-117: on the inner interfaces the WENO7-Z value w
+// (eps 1e-20) blended with the 8-point central value q8 through
+// theta = 1/(1 + X^2), i.e. (X^2 w + q8)/(1 + X^2); on the edge interfaces w
+// alone (:207-304).  One WENO7-Z evaluation serves both.
 // f[0..7]: one downwind point more than WENO7.
 template <typename T, typename TW>
-__device__ __forceinline__ TW hccs78_inner(const T *f)
+__device__ __forceinline__ TW hccs78_value(const T *f, bool edge)
 {
-    TW asum;
-    TW w = weno7z<T, TW>(f, TW(1.0e-20), asum);
-    TW q8 = (TW(-3) * (TW(f[7]) + TW(f[0])) + TW(29) * (TW(f[6]) + TW(f[1])) - TW(139) * (TW(f[5]) + TW(f[2]))
-             + TW(533) * (TW(f[4]) + TW(f[3]))) / TW(840);
-    TW theta = TW(1) / (TW(1) + sq(asum - TW(1)));
-    return (TW(1) - theta) * w + theta * q8;
+    TW X;
+    const TW w = weno7z<T, TW>(f, TW(1.0e-20), X);
+    const TW q8 = (TW(-3) * (TW(f[7]) + TW(f[0])) + TW(29) * (TW(f[6]) + TW(f[1])) - TW(139) * (TW(f[5]) + TW(f[2]))
+                   + TW(533) * (TW(f[4]) + TW(f[3]))) * TW(1.0 / 840.0);
+    const TW theta = frcp(TW(1) + sq(X));
+    return edge ? w : w + theta * (q8 - w);
 }
 
-// hccs77 interior row, src/hccs77.cpp:86-163: WENO7-Z (eps 1e-20) and the
-// 7th-order upwind compact row blended through theta = 1/(1 + (asum-1)^2);
-// theta > 0.5 keeps the compact row alone.  f[0..6]; TW: weights and the row.
+// hccs77 row, src/hccs77.cpp:86-163 (explicit rows :349-455): the 7th-order
+// upwind compact row, and where theta = 1/(1 + X^2) <= 0.5 (X >= 1) its blend
+// with the explicit WENO7-Z row w.  Every row is scaled by 1 + X^2 = 1/theta,
+// which leaves the solution unchanged: compact row + X^2 (x = w).
+// f[0..6]; TW: weights and the row.
 template <typename T, typename TW>
-__device__ __forceinline__ void hccs77_row(const T *f, TW &lo, TW &di, TW &hi, TW &rhs)
+__device__ __forceinline__ void hccs77_row(const T *f, bool expl, TW &lo, TW &di, TW &hi, TW &rhs)
 {
-    TW asum;
-    TW w = weno7z<T, TW>(f, TW(1.0e-20), asum);
-    TW q7 = (-TW(f[1]) + TW(19) * TW(f[2]) + TW(239) * TW(f[3]) + TW(159) * TW(f[4]) + TW(4) * TW(f[5])) / TW(420);
-    TW theta = TW(1) / (TW(1) + sq(asum - TW(1)));
-    if (theta > TW(0.5)) {
-        lo = TW(2.0 / 7.0); di = TW(4.0 / 7.0); hi = TW(1.0 / 7.0); rhs = q7;
-    } else {
-        lo = TW(2.0 / 7.0) * theta;
-        di = TW(1) + (TW(4.0 / 7.0) - TW(1)) * theta;
-        hi = TW(1.0 / 7.0) * theta;
-        rhs = w * (TW(1) - theta) + q7 * theta;
-    }
+    TW X;
+    const TW w = weno7z<T, TW>(f, TW(1.0e-20), X);
+    const TW q7 = (-TW(f[1]) + TW(19) * TW(f[2]) + TW(239) * TW(f[3]) + TW(159) * TW(f[4]) + TW(4) * TW(f[5])) * TW(1.0 / 420.0);
+    const TW s = X < TW(1) ? TW(0) : sq(X);
+    lo = expl ? TW(0) : TW(2.0 / 7.0);
+    di = expl ? TW(1) : TW(4.0 / 7.0) + s;
+    hi = expl ? TW(0) : TW(1.0 / 7.0);
+    rhs = expl ? w : q7 + s * w;
 }
 
 // WENO3-JS, src/weno3js.cpp:80-93 (eps 1e-6): f[0..2] upwind
@@ -143,6 +172,11 @@ __device__ __forceinline__ TW weno3js(const T *f)
 // hccs interior row, src/hccs.cpp:138-183: Z-type CRWENO weights (eps 1e-40)
 // blended with the 7th-order upwind compact scheme through theta.
 // T: indicators and stencil values; TW: weights and the row.
+// With S_k = (is_k + eps)^2 the unnormalised weights are c_k (S_k + tau^2)/S_k.
+// Their sum less 1 is X = tau^2 sum_k c_k prod_{j!=k} S_j / (S_0 S_1 S_2),
+// theta = 1/(1 + X^2) and the CRWENO row's factor (1 - theta)/theta = X^2:
+// two reciprocals in place of seven quotients.  The products hold indicators
+// between 1e-40 and 1e50 (fluxes up to about 1e25).
 template <typename T, typename TW>
 __device__ __forceinline__ void hccs_row(T f0, T f1, T f2, T f3, T f4, TW &lo, TW &di, TW &hi, TW &rhs)
 {
@@ -151,26 +185,21 @@ __device__ __forceinline__ void hccs_row(T f0, T f1, T f2, T f3, T f4, TW &lo, T
     T is0 = g0 * sq(f0 - T(2) * f1 + f2) + g1 * sq(f0 - T(4) * f1 + T(3) * f2);
     T is1 = g0 * sq(f1 - T(2) * f2 + f3) + g1 * sq(f1 - f3);
     T is2 = g0 * sq(f2 - T(2) * f3 + f4) + g1 * sq(T(3) * f2 - T(4) * f3 + f4);
-    T q7 = (-f0 + T(19) * f1 + T(239) * f2 + T(159) * f3 + T(4) * f4) / T(420);
-    const TW b0 = is0, b1 = is1, b2 = is2;
-    TW tau = fabs(b2 - b0);
-    TW a0 = TW(0.2) * (TW(1) + sq(tau / (b0 + eps)));
-    TW a1 = TW(0.5) * (TW(1) + sq(tau / (b1 + eps)));
-    TW a2 = TW(0.3) * (TW(1) + sq(tau / (b2 + eps)));
-    TW asum = a0 + a1 + a2;
-    TW theta = TW(1) / (TW(1) + sq(asum - TW(1)));
-    if (theta > TW(0.5)) {
-        lo = TW(2.0 / 7.0); di = TW(4.0 / 7.0); hi = TW(1.0 / 7.0); rhs = q7;
-    } else {
-        TW r = TW(1) / asum;
-        TW w0 = a0 * r, w1 = a1 * r, w2 = a2 * r;
-        TW s = (TW(1) - theta) / theta;
-        TW F1 = f1, F2 = f2, F3 = f3;
-        lo = (TW(2.0 / 3.0) * w0 + TW(1.0 / 3.0) * w1) * s + TW(2.0 / 7.0);
-        di = (TW(1.0 / 3.0) * w0 + TW(2.0 / 3.0) * (w1 + w2)) * s + TW(4.0 / 7.0);
-        hi = (TW(1.0 / 3.0) * w2) * s + TW(1.0 / 7.0);
-        rhs = ((w0 * F1 + (TW(5) * (w0 + w1) + w2) * F2 + (w1 + TW(5) * w2) * F3) * TW(1.0 / 6.0)) * s + TW(q7);
-    }
+    T q7 = (-f0 + T(19) * f1 + T(239) * f2 + T(159) * f3 + T(4) * f4) * T(1.0 / 420.0);
+    const TW S0 = sq(TW(is0) + eps), S1 = sq(TW(is1) + eps), S2 = sq(TW(is2) + eps);
+    const TW T2 = sq(TW(is2) - TW(is0));
+    const TW P12 = S1 * S2;
+    const TW p0 = TW(0.2) * P12, p1 = TW(0.5) * (S0 * S2), p2 = TW(0.3) * (S0 * S1);
+    const TW X = (T2 * (p0 + p1 + p2)) * frcp(S0 * P12);
+    const TW n0 = (S0 + T2) * p0, n1 = (S1 + T2) * p1, n2 = (S2 + T2) * p2;
+    // theta > 0.5 (X < 1): the compact row alone
+    const TW s = X < TW(1) ? TW(0) : sq(X) * frcp(n0 + n1 + n2);
+    const TW w0 = n0 * s, w1 = n1 * s, w2 = n2 * s;
+    const TW F1 = f1, F2 = f2, F3 = f3;
+    lo = (TW(2.0 / 3.0) * w0 + TW(1.0 / 3.0) * w1) + TW(2.0 / 7.0);
+    di = (TW(1.0 / 3.0) * w0 + TW(2.0 / 3.0) * (w1 + w2)) + TW(4.0 / 7.0);
+    hi = TW(1.0 / 3.0) * w2 + TW(1.0 / 7.0);
+    rhs = (w0 * F1 + (TW(5) * (w0 + w1) + w2) * F2 + (w1 + TW(5) * w2) * F3) * TW(1.0 / 6.0) + TW(q7);
 }
 
 }  // namespace nucdev

@@ -29,18 +29,6 @@ struct Zone {
     int off = 0;  // position of interface 0 on the full line (a segment of a long line)
 };
 
-// reciprocal: hardware estimate refined by two Newton steps (|err| <= 1 ulp)
-__device__ __forceinline__ double frcp(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
-}
-// FP32 (mixed path): the hardware reciprocal, 1 ulp
-__device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
-
 // Unnormalised WENO5 weights n_k ~ c_k / (eps + is_k)^2.  FP64 uses the
 // division-free products c_k * s_i * s_j (one reciprocal per row in total);
 // FP32 uses c_k * rcp(s_k), since the products can leave FP32's range.
@@ -318,12 +306,16 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             // 13/12 (f2 - f3)^2 in place of its second-difference term
             bool typo = !neg && ml[r] >= z.ts && ml[r] <= z.nloc - z.ts;
             if (typo) b2 = T(13.0 / 12.0) * sq(d3) + h2 * h2;
+            // alpha_k = c_k (1 + (tau/s_k)^2), s_k = is_k + eps (src/weno5z.cpp:84-92),
+            // scaled by s_0^2 s_1^2 s_2^2: no quotient is left but the normalisation
+            // (three IEEE quotients are 35 of the plain form's 75 instructions).  The
+            // products hold indicators between eps = 1e-40 and 1e50.
             const TW eps = TW(1.0e-40);
             const TW B0 = b0, B1 = b1, B2 = b2;
-            TW tau = fabs(B2 - B0);
-            TW a0 = TW(0.1) * (TW(1) + sq(tau / (B0 + eps)));
-            TW a1 = TW(0.6) * (TW(1) + sq(tau / (B1 + eps)));
-            TW a2 = TW(0.3) * (TW(1) + sq(tau / (B2 + eps)));
+            const TW S0 = sq(B0 + eps), S1 = sq(B1 + eps), S2 = sq(B2 + eps), T2 = sq(B2 - B0);
+            const TW a0 = TW(0.1) * ((S0 + T2) * (S1 * S2));
+            const TW a1 = TW(0.6) * ((S1 + T2) * (S0 * S2));
+            const TW a2 = TW(0.3) * ((S2 + T2) * (S0 * S1));
             TS o = TS((a0 * TW(q0) + a1 * TW(q1) + a2 * TW(q2)) * frcp(a0 + a1 + a2));
             pin(o); pin(f3); pin(f4); pin(d3); pin(d4); pin(e2); pin(e3);
             out[r] = o;
@@ -362,7 +354,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         for (int r = 0; r < R; r++) {
             fw[7] = win[r + 7];
             bool edge = ml[r] < z.ts || ml[r] > z.nloc - z.ts;
-            TS o = edge ? TS(weno7z<T, TW>(fw, TW(1.0e-20))) : TS(hccs78_inner<T, TW>(fw));
+            TS o = TS(hccs78_value<T, TW>(fw, edge));
             pin(o);
 #pragma unroll
             for (int j = 1; j < 8; j++) pin(fw[j]);
@@ -439,11 +431,9 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             int m = m0r + mstep * r;
             bool valid = full || m < z.nrows;
             bool expl = ml[r] <= z.ts || ml[r] >= z.nloc - z.ts;
-            TW a = TW(0), b = TW(1), c = TW(0), d = TW(0);
-            if (valid) {
-                if (expl) d = weno7z<T, TW>(f, TW(1.0e-20));
-                else hccs77_row<T, TW>(f, a, b, c, d);
-            }
+            TW a, b, c, d;
+            hccs77_row<T, TW>(f, expl, a, b, c, d);
+            if (!valid) { a = TW(0); b = TW(1); c = TW(0); d = TW(0); }
             TS as = TS(a), bs = TS(b), cs = TS(c), ds = TS(d);
             if (r > 0) {
                 pin(ch.Af[r - 1]); pin(ch.Cf[r - 1]); pin(ch.Df[r - 1]);
@@ -460,6 +450,29 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         for (int r = 0; r < R; r++) out[r] = ch.Df[r];
     } else {  // HCCS
         Chunk<R, TS> ch;
+        // The explicit WENO7-Z rows (2 ts + 1 around every rank-block edge) lie
+        // in a few lanes only.  Evaluated in the row loop, all R rows of every
+        // wave pay for them (about 150 instructions each).  Lines of up to two
+        // blocks have at most 27 of them: lane h evaluates the h-th, and leaves
+        // its value at the interface's place in the line buffer, whose windows
+        // are in registers by then.
+        T *const Lb = const_cast<T *>(Lw) - h * (R + 1);
+        const int ne = 2 * z.ts + 1, nexp = (z.nrows / z.nloc + 1) * ne;
+        const bool ahead = nexp <= 32;
+        if (ahead) {
+            const int e = h / ne, m = e * z.nloc + (h - e * ne) - z.ts;   // interface of the h-th row
+            const bool mine = h < nexp && m >= 0 && m < z.nrows;
+            const int y = !mine ? 0 : (neg ? 32 * R - 1 - m : m);         // its position in the lane order
+            T fe[7];
+#pragma unroll
+            for (int j = 0; j < 7; j++) fe[j] = Lb[Skew<R>::at(y - 4 + j)];
+            TW x = weno7z<T, TW>(fe, TW(1.0e-40));
+            pin(x);
+#pragma unroll
+            for (int t = 0; t < W; t++) pin(win[t]);
+            if (mine) Lb[Skew<R>::at(y)] = T(x);
+            __builtin_amdgcn_wave_barrier();
+        }
         T fw[7];   // 7-point window for the closures, 5-point from fw+1
 #pragma unroll
         for (int j = 0; j < 6; j++) fw[j] = win[j];
@@ -470,14 +483,10 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             int m = m0r + mstep * r;
             bool valid = full || m < z.nrows;
             bool expl = ml[r] <= z.ts || ml[r] >= z.nloc - z.ts;
-            TW a = TW(0), b = TW(1), c = TW(0), d = TW(0);
-            if (valid) {
-                if (expl) {
-                    d = weno7z<T, TW>(f, TW(1.0e-40));
-                } else {
-                    hccs_row<T, TW>(f[1], f[2], f[3], f[4], f[5], a, b, c, d);
-                }
-            }
+            TW a, b, c, d, x = TW(Lw[Skew<R>::at(r)]);
+            if (!ahead && valid && expl) x = weno7z<T, TW>(f, TW(1.0e-40));
+            hccs_row<T, TW>(f[1], f[2], f[3], f[4], f[5], a, b, c, d);
+            if (expl || !valid) { a = TW(0); b = TW(1); c = TW(0); d = valid ? x : TW(0); }
             TS as = TS(a), bs = TS(b), cs = TS(c), ds = TS(d);
             if (r > 0) {
                 pin(ch.Af[r - 1]); pin(ch.Cf[r - 1]); pin(ch.Df[r - 1]);

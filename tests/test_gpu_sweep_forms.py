@@ -1,0 +1,61 @@
+"""The sweep kernel's forms at the sizes where their rules change, one RHS
+evaluation each against the oracle (NaiverStokesData3d::solve,
+src/NaiverStokes3d.cpp:37-73).  The bars are those of test_gpu_rhs.py: 1e-11
+relative per conserved variable, and for the schemes with cancelling 7-point
+indicators three times the oracle's own change under +-1 ulp of its input."""
+import numpy as np
+import pytest
+
+import nuc3d_amd as G
+import oracle as O
+from test_gpu_rhs import ILL_CONDITIONED, _ulp_floor
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # n, rank grid, scheme, viscous scheme, splitting
+    # hccs explicit rows evaluated ahead of the row loop (up to 2 blocks a
+    # line) and inside it (3 and more); 10 cells is the shortest block
+    ((10, 20, 30), (1, 2, 3), G.HCCS, G.CD6, G.AUSM),
+    ((30, 10, 20), (3, 1, 2), G.HCCS, G.CD8, G.LF),
+    ((12, 66, 33), (1, 3, 3), G.HCCS, G.CD6, G.AUSMP),
+    # one WENO7-Z evaluation for both kinds of row
+    ((10, 20, 30), (1, 2, 3), G.HCCS77, G.CD6, G.AUSM),
+    ((10, 20, 30), (1, 2, 3), G.HCCS78, G.CD8, G.LF),
+]
+
+
+def _state(oc, seed):
+    """Taylor-Green with a seeded 3-D perturbation: every variable of order one."""
+    q = O.init_tgv(oc)
+    N = oc.nx * oc.ny * oc.nz
+    rng = np.random.default_rng(seed)
+    q = q.reshape(5, N)
+    q[3] += 0.2 * np.sin(np.linspace(0, 40, N) + rng.random())
+    q[0] *= 1.0 + 0.01 * rng.standard_normal(N)
+    return q.ravel().copy()
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}-s{c[2]}-v{c[3]}-r{c[4]}")
+def test_rhs_matches_oracle(case):
+    n, npr, scheme, vis, rie = case
+    print(f"sweep form {case}", flush=True)
+    kw = dict(n=n, npr=npr, scheme=scheme, vis=vis, riemann=rie, model=G.NAVIERSTOKES3D)
+    gc, oc = G.make_config(**kw), O.make_config(**kw)
+    oc.nthreads = 8
+    q = _state(oc, 11)
+    N = oc.nx * oc.ny * oc.nz
+    s = O.Solver(oc)
+    s.set_state(q)
+    ref, dt_ref = s.rhs()
+    with G.Context(gc) as ctx:
+        ctx.upload(q)
+        got, dt = ctx.rhs()
+    ref, got = ref.reshape(5, N), got.reshape(5, N)
+    err = np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)
+    tol = np.full(5, 1e-11)
+    if scheme in ILL_CONDITIONED:
+        tol = np.maximum(tol, 3.0 * _ulp_floor(oc, q, 0))
+    print("rel err", err, "tol", tol, flush=True)
+    assert np.all(err <= tol), (err, tol)
+    assert abs(dt - dt_ref) <= 1e-14 * dt_ref
