@@ -584,26 +584,29 @@ int rows_for(int nrows)
     return -1;
 }
 
+// Waves per line of a sweep: one (32 lanes per sign) up to 256 cells; above,
+// two (one per sign, 64 lanes each), which halves the rows a lane holds: on
+// one wave a 512-cell line takes 16 rows a lane, whose 257 registers (or 103
+// KB of LDS) leave one wave per SIMD.  Measured, ms a sweep on one -> two
+// waves: 512^3 hccs/AUSM x 17.9 -> 11.2, 512x256^2 CRWENO5 x 3.39 -> 1.98,
+// 512x128^2 WENO5-Z/AUSM x 0.51 -> 0.40, 384x64x384 WENO5-JS z 0.48 -> 0.47.
+// With FP32 stencils (half the LDS and registers) the y and z sweeps stay on
+// one wave, where the larger workgroup's barriers cost more than it gains:
+// 384x64x384 mixed CRWENO5 z 0.47 against 0.53, x 0.51 -> 0.45.
+int sweep_wpl(int n, int dir, bool fp32_stencils) { return n > 256 && (dir == 0 || !fp32_stencils) ? 2 : 1; }
+
 // rows per lane of a sweep over a periodic line of n cells: also 3 and 5, so
-// that lines of 65-96 and 129-160 cells do not leave up to a quarter of the
-// lanes idle, and 12 for 289-384 cells (on 16 rows a 384-cell line leaves a
-// quarter idle, and the compact schemes' workgroups hold 103 KB of LDS, one
-// per CU, against 77 KB).  7 rows for 193-224 cells measured no faster than
-// 8 (odd R has no affine LDS slots and no tail-free form).
-int sweep_rows(int n)
+// that lines of 65-96 and 129-160 cells (257-320 on two waves) do not leave up
+// to a quarter of the lanes idle, and 12 for 289-384 cells on one wave.  7 rows
+// for 193-224 cells measured no faster than 8 (odd R has no affine LDS slots
+// and no tail-free form).
+int sweep_rows(int n, int wpl)
 {
-    int r = (n + 31) / 32;
+    const int lanes = 32 * wpl, r = (n + lanes - 1) / lanes;
     if (r == 3 || r == 5) return r;
     if (r >= 10 && r <= 12) return 12;
-    return rows_for(n);
+    return rows_for(32 * r);
 }
-
-// lines per workgroup: 4 (one wave per line).  With the sweep's register
-// budget two such workgroups share a CU, so one workgroup's barrier waits
-// overlap the other's work; the y/z load mapping still reads 4 consecutive
-// x cells per line cell, and xcd_block keeps the neighbouring groups that
-// share the cache line on one XCD.
-int sweep_lpb(int) { return SWEEP_LPB; }
 
 void launch_sweep(int scheme, int R, const SweepArgs &A, hipStream_t s)
 {
@@ -695,6 +698,7 @@ struct nuc_ctx {
     hipStream_t stream = nullptr;
     long N = 0;
     int n[3], np[3], nloc[3], ts[3], tsv[3], cpt[3];
+    int wpl[3];            // waves per line of the sweeps (cpt rows per lane)
     int seg[3], nseg[3];   // sweep segment length and count per line (nseg = 1 up to 512 cells)
     double h[3];
     int P = 1;
@@ -905,7 +909,10 @@ static void ctx_geometry(nuc_ctx *x, const nuc_config *cfg)
         x->tsv[d] = vis_tilesize(cfg->scheme[d], cfg->vis_scheme[d]);
         x->seg[d] = segment_length(x->n[d], x->nloc[d], x->np[d], cfg->scheme[d]);
         x->nseg[d] = x->n[d] / x->seg[d];
-        x->cpt[d] = x->nseg[d] > 1 ? (x->seg[d] <= 255 ? 8 : 16) : sweep_rows(x->n[d]);
+        // a segment has seg + 1 interfaces: at most 256, or 512 (compact schemes) on two waves
+        const bool f32s = cfg->precision != NUC_FP64 && cfg->scheme[d] != NUC_HCCS && cfg->scheme[d] != NUC_HCCS77;
+        x->wpl[d] = x->nseg[d] > 1 ? (x->seg[d] > 255 ? 2 : 1) : sweep_wpl(x->n[d], d, f32s);
+        x->cpt[d] = x->nseg[d] > 1 ? 8 : sweep_rows(x->n[d], x->wpl[d]);
     }
 }
 
@@ -975,7 +982,8 @@ extern "C" int nuc_create(const nuc_config *cfg, nuc_ctx **out)
     // residual partials: one per workgroup of the last sweep
     const int dl = kSweepOrder[2];
     long lines_last = x->N / x->n[dl] * x->nseg[dl];
-    x->res_nb = (lines_last + sweep_lpb(x->cpt[dl]) - 1) / sweep_lpb(x->cpt[dl]);
+    const int lpb_last = sweep_lpb(x->wpl[dl], dl, cfg->scheme[dl]);
+    x->res_nb = (lines_last + lpb_last - 1) / lpb_last;
     if (!dalloc(&x->res_part, x->res_nb * sizeof(double))) return fail("device allocation (residual)");
     (void)hipMemsetAsync(x->lam, 0, 3 * MAXRANK * sizeof(unsigned long long), x->stream);
     (void)hipMemsetAsync(x->scal, 0, 8 * sizeof(double), x->stream);
@@ -1144,6 +1152,7 @@ static void stage_args(nuc_ctx *x, int in, int stage, int outb, bool epilogue, S
         const bool first = (d == kSweepOrder[0]), last = (d == kSweepOrder[2]);
         S.first = first ? 1 : 0;
         S.accum = (first && (x->forcing || x->sources)) ? 1 : 0;
+        S.wpl = x->wpl[d];
         S.mixed = x->mixed ? 1 : 0;
         S.fp32 = x->fp32 ? 1 : 0;
         S.fv_f32 = x->fv32 ? 1 : 0;   // k_gradq<float>

@@ -55,7 +55,7 @@ template <int SCH> struct Extra { static constexpr int value = (SCH == HCCS78) ?
 // Skewed LDS line layout: position y (y >= -B) lives at slot (y+B) + (y+B)/R,
 // one pad slot after every R positions, B = HALO+1 rounded up to a multiple of
 // R.  The f^+ line stores cell x at y = x; the f^- line is stored mirrored,
-// y = 32R-2-x, so that both half waves read their windows upwards from
+// y = NL R-2-x (NL lanes per sign), so that both signs read their windows upwards from
 // y = hR-RAD-1: the lane's window then starts at slot h*(R+1) + at(-RAD-1)
 // and every window element is a compile-time offset from one base.  Lanes R
 // positions apart sit R+1 slots apart (odd), so chunk reads and the
@@ -63,10 +63,10 @@ template <int SCH> struct Extra { static constexpr int value = (SCH == HCCS78) ?
 // pitch(): line stride in slots, = 4 (mod 16): the y/z load mapping writes 4
 // lines x 4 consecutive cells per 16 lanes, which then hit distinct banks
 // (measured: y/z sweep bank-conflict cycles -79% against a pitch = 2 mod 16).
-template <int R> struct Skew {
+template <int R, int NL = 32> struct Skew {
     static constexpr int B = ((HALO + 1 + R - 1) / R) * R;
     __host__ __device__ static constexpr int at(int y) { return (y + B) + (y + B) / R; }
-    __device__ __forceinline__ static int mir(int x) { return at(32 * R - 2 - x); }
+    __device__ __forceinline__ static int mir(int x) { return at(NL * R - 2 - x); }
     // slots up to cell ncap+HALO: the last one is a write-only dummy (halo
     // writes of interior cells go there instead of branching)
     static constexpr int span(int ncap) { return at(ncap + HALO) + 1; }
@@ -129,24 +129,43 @@ __device__ __forceinline__ void swap16(float x, float &up, float &dn)
 // statements keep their order).  Used to evaluate a lane's rows in order.
 template <typename T> __device__ __forceinline__ void pin(T &x) { asm volatile("" : "+v"(x)); }
 
-// normalised parallel cyclic reduction over the 32 lanes of a half wave:
-// row k: x_k + al*x_{k-1} + ga*x_{k+1} = de  ->  x_k = de on return
-template <typename T>
-__device__ __forceinline__ void pcr32(T &al, T &ga, T &de, int h)
+// Distance-32 exchange between the two halves of a wave (v_permlane32_swap):
+// up is meaningful for lanes >= 32 (the value of lane i-32), dn for lanes < 32
+// (lane i+32).
+__device__ __forceinline__ void swap32(unsigned x, unsigned &up, unsigned &dn)
+{
+    auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    up = r[0]; dn = r[1];
+}
+__device__ __forceinline__ void swap32(double x, double &up, double &dn)
+{
+    unsigned hu, hd, lu, ld;
+    swap32((unsigned)__double2hiint(x), hu, hd);
+    swap32((unsigned)__double2loint(x), lu, ld);
+    up = __hiloint2double((int)hu, (int)lu);
+    dn = __hiloint2double((int)hd, (int)ld);
+}
+
+// normalised parallel cyclic reduction over the NL lanes (32 or 64) of one
+// sign: row k: x_k + al*x_{k-1} + ga*x_{k+1} = de  ->  x_k = de on return
+template <int NL, typename T>
+__device__ __forceinline__ void pcr(T &al, T &ga, T &de)
 {
 #pragma unroll
-    for (int s = 1; s < 32; s <<= 1) {
+    for (int s = 1; s < NL; s <<= 1) {
         T alm, gam, dem, alp, gap, dep;
         if (s == 1) {
             alm = shr1(al); gam = shr1(ga); dem = shr1(de);
             alp = shl1(al); gap = shl1(ga); dep = shl1(de);
-        } else if (s == 16) {
+        } else if (s == 16 && NL == 32) {
             swap16(al, alm, alp); swap16(ga, gam, gap); swap16(de, dem, dep);
+        } else if (s == 32) {
+            swap32(al, alm, alp); swap32(ga, gam, gap); swap32(de, dem, dep);
         } else {
-            alm = __shfl_up(al, s, 32); gam = __shfl_up(ga, s, 32); dem = __shfl_up(de, s, 32);
-            alp = __shfl_down(al, s, 32); gap = __shfl_down(ga, s, 32); dep = __shfl_down(de, s, 32);
+            alm = __shfl_up(al, s, NL); gam = __shfl_up(ga, s, NL); dem = __shfl_up(de, s, NL);
+            alp = __shfl_down(al, s, NL); gap = __shfl_down(ga, s, NL); dep = __shfl_down(de, s, NL);
         }
-        // no masks: lanes h < s hold al = 0 and lanes h + s >= 32 hold ga = 0
+        // no masks: lanes h < s hold al = 0 and lanes h + s >= NL hold ga = 0
         // exactly (the first and last rows do not couple outward, and each
         // level doubles those ranges), so the values they received from the
         // wrapped or neighbouring lanes, all finite, are multiplied by zero
@@ -160,7 +179,7 @@ __device__ __forceinline__ void pcr32(T &al, T &ga, T &de, int h)
 
 // Forward-eliminated rows of one lane's chunk (rows normalised):
 //   r = 0: Af x_{-1} + x_0 + Cf x_1 = Df ;  r >= 1: Af x_0 + x_r + Cf x_{r+1} = Df
-template <int R, typename T> struct Chunk {
+template <int R, typename T, int NL> struct Chunk {
     T Af[R], Cf[R], Df[R];
     __device__ __forceinline__ void row(int r, T a, T b, T c, T d)
     {
@@ -174,8 +193,8 @@ template <int R, typename T> struct Chunk {
             Cf[r] = rr * c;
         }
     }
-    // Partition solve across the half wave (lane h holds chunk h in system
-    // order; the first row of lane 0 and the last row of lane 31 must not
+    // Partition solve across the NL lanes of a sign (lane h holds chunk h in system
+    // order; the first row of lane 0 and the last row of lane NL-1 must not
     // couple outward).  Solution returned in Df.  Equivalent to the
     // reference's Thomas sweep (src/crweno5.cpp:208-219) up to rounding.
     __device__ __forceinline__ void solve(int h)
@@ -198,15 +217,15 @@ template <int R, typename T> struct Chunk {
         }
         T A1 = Af[R - 1], C1 = Cf[R - 1], D1 = Df[R - 1];
         T A0n = shl1(A0), C0n = shl1(C0), D0n = shl1(D0);
-        if (h == 31) { A0n = T(0); C0n = T(0); D0n = T(0); }
+        if (h == NL - 1) { A0n = T(0); C0n = T(0); D0n = T(0); }
         T rb = frcp(T(1) - A1 * C0 - C1 * A0n);
         T al = -rb * A1 * A0;
         T ga = -rb * C1 * C0n;
         T de = rb * (D1 - A1 * D0 - C1 * D0n);
         // the reduced system's first and last rows do not couple outward
         if (h == 0) al = T(0);
-        if (h == 31) ga = T(0);
-        pcr32(al, ga, de, h);
+        if (h == NL - 1) ga = T(0);
+        pcr<NL>(al, ga, de);
         T X1 = de;
         T X1m = shr1(X1);
         if (h == 0) X1m = T(0);
@@ -247,8 +266,9 @@ __device__ __forceinline__ void w5_diff(T f2, T f3, T d1, T d2, T d3, T d4, T e1
 // T is the type of the stencils (smoothness indicators, candidate values);
 // TW the type of the nonlinear weights and compact rows; TS the type of the
 // tridiagonal solve and of the result (FP64 in both precision paths).
-// full: every row of every lane is an interface of the line (n = 32R).
-template <int SCH, int R, typename T, typename TW, typename TS>
+// NL: lanes per sign, h in [0, NL).
+// full: every row of every lane is an interface of the line (n = NL R).
+template <int SCH, int R, typename T, typename TW, typename TS, int NL = 32>
 __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const Zone &z, int h, bool neg,
                                           TS out[R], bool full = false)
 {
@@ -363,7 +383,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             for (int j = 0; j < 7; j++) fw[j] = fw[j + 1];
         }
     } else if constexpr (SCH == CRWENO5) {
-        Chunk<R, TS> ch;
+        Chunk<R, TS, NL> ch;
         // Rows in order: a rolling window (f1..f4, the differences d1..d4 and
         // the second-difference terms e1..e3 of the current row), where the
         // values the next row reuses and the row's own coefficients pass
@@ -420,7 +440,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
     } else if constexpr (SCH == HCCS77) {
         // compact rows on ts+1..nloc-ts-1, WENO7-Z rows at ts and nloc-ts and
         // on the edges (src/hccs77.cpp:86-163, :349-455)
-        Chunk<R, TS> ch;
+        Chunk<R, TS, NL> ch;
         T fw[7];
 #pragma unroll
         for (int j = 0; j < 6; j++) fw[j] = win[j];
@@ -449,7 +469,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
 #pragma unroll
         for (int r = 0; r < R; r++) out[r] = ch.Df[r];
     } else {  // HCCS
-        Chunk<R, TS> ch;
+        Chunk<R, TS, NL> ch;
         // The explicit WENO7-Z rows (2 ts + 1 around every rank-block edge) lie
         // in a few lanes only.  Evaluated in the row loop, all R rows of every
         // wave pay for them (about 150 instructions each).  Lines of up to two
@@ -458,11 +478,11 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // are in registers by then.
         T *const Lb = const_cast<T *>(Lw) - h * (R + 1);
         const int ne = 2 * z.ts + 1, nexp = (z.nrows / z.nloc + 1) * ne;
-        const bool ahead = nexp <= 32;
+        const bool ahead = nexp <= NL;
         if (ahead) {
             const int e = h / ne, m = e * z.nloc + (h - e * ne) - z.ts;   // interface of the h-th row
             const bool mine = h < nexp && m >= 0 && m < z.nrows;
-            const int y = !mine ? 0 : (neg ? 32 * R - 1 - m : m);         // its position in the lane order
+            const int y = !mine ? 0 : (neg ? NL * R - 1 - m : m);         // its position in the lane order
             T fe[7];
 #pragma unroll
             for (int j = 0; j < 7; j++) fe[j] = Lb[Skew<R>::at(y - 4 + j)];

@@ -57,6 +57,7 @@ struct SweepArgs {
     int stage, epilogue;
     int first;                // the stage's first sweep: writes rhs without reading it
     int accum;                // the first sweep adds to rhs (forcing initialised it)
+    int wpl;                  // waves per line: 1, or 2 (one per sign; host-side dispatch only)
     int mixed;                // FP32 stencils (host-side dispatch only)
     int fp32;                 // FP32 state and RHS (NUC_FP32; host-side dispatch only)
     const double GMEM *fmean; // last sweep: <f.u> added back to the energy RHS
@@ -183,9 +184,10 @@ __device__ __forceinline__ void sync_wave()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+template <int WPL>
 __device__ __forceinline__ void sync_lines(int d)
 {
-    if (d == 0) sync_wave();
+    if (WPL == 1 && d == 0) sync_wave();
     else __syncthreads();
 }
 
@@ -203,12 +205,15 @@ __device__ __forceinline__ void sync_lines(int d)
 // whole line; the 2*HALO cells around the segment are read from the
 // neighbouring segments (periodic over the full line) and the segment's n+1
 // interfaces are all computed, so that no periodic image is needed.
-template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false>
+template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1>
 __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
 {
     const bool epi = EPI == EPI_ARG ? A.epilogue != 0 : EPI == EPI_YES;
-    constexpr int NP = Skew<R>::pitch(32 * R);
-    constexpr int NV = plain_pitch(32 * R);
+    constexpr int NL = 32 * WPL;           // lanes per sign
+    using Sk = Skew<R, NL>;
+    constexpr int GS = 64 * WPL;           // threads per line in the load mapping
+    constexpr int NP = Sk::pitch(NL * R);
+    constexpr int NV = plain_pitch(NL * R);
     constexpr int CPL = (R + 1) / 2;       // cells per thread in the load mapping (odd R: the last slot of
                                            // the upper half-wave is past the line)
     constexpr int NSP = (RIE == RIE_LF) ? 3 : 5;
@@ -218,11 +223,11 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     __shared__ double sP[LPB * NP];
     __shared__ double sM[LPB * NP];
     __shared__ T sV[LPB * NV];
-    __shared__ double sRed[LPB];
+    __shared__ double sRed[LPB * WPL];
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int n = A.n, d = A.dir;   // SEG: n is the segment length
     int ll, g;
-    if (d == 0) { ll = wave; g = lane; }
+    if (d == 0) { ll = t / GS; g = t % GS; }
     else { ll = t % LPB; g = t / LPB; }
     const long L = blk * LPB + ll;   // SEG: the segment L % nseg of line L / nseg
     const long nll = SEG ? A.nlines * A.nseg : A.nlines;
@@ -243,7 +248,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     // field's base address (uniform, in scalar registers) plus this offset
     unsigned ob[CPL];
 #pragma unroll
-    for (int k = 0; k < CPL; k++) ob[k] = (unsigned)(base + (long)(g + 64 * k) * stride) * 8u;
+    for (int k = 0; k < CPL; k++) ob[k] = (unsigned)(base + (long)(g + GS * k) * stride) * 8u;
     // bytes of one FP64 field (the buffer's bound: 2^32 - 1 at the largest box)
     const unsigned fb = (unsigned)std::min<long>((long)A.nlines * (SEG ? A.nfull : n) * 8, 0xFFFFFFFFl);
     // state and RHS fields hold S (ob, fb are for 8-byte elements)
@@ -262,12 +267,12 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     // explicit schemes keep them in CPL*NSP registers: with the LDS copy the
     // workgroup's 53 KB (LF) would allow only three workgroups per CU.
     constexpr bool SP_LDS = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
-    __shared__ T sSP[SP_LDS ? CPL * NSP : 1][SP_LDS ? 64 * LPB : 1];
+    __shared__ T sSP[SP_LDS ? CPL * NSP : 1][SP_LDS ? GS * LPB : 1];
     T spr[SP_LDS ? 1 : CPL][SP_LDS ? 1 : NSP];
     unsigned innermask = 0;   // cd8 inner-form cells (rank-local position)
 #pragma unroll
     for (int k = 0; k < CPL; k++) {
-        int c = g + 64 * k;
+        int c = g + GS * k;
         bool ok = FULL || (lv && c < n);
         T q[5];
 #pragma unroll
@@ -301,37 +306,38 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         split_params<RIE, T>(q, d, T(A.gamma), sph, A.riemann == RIE_AUSMP);
     }
 
-    // f^+ / f^- line buffers (skewed, f^- mirrored: Skew<R>::at / mir) and the
+    // f^+ / f^- line buffers (skewed, f^- mirrored: Sk::at / mir) and the
     // plain viscous-flux line
     // a line's T view lives inside the bytes of its own double line, so that
     // in the x sweep (wave-level sync only) no wave's writes reach another's line
     T *Pl = reinterpret_cast<T *>(sP + ll * NP), *Ml = reinterpret_cast<T *>(sM + ll * NP);
     T *Vl = sV + ll * NV + HALO;
-    double *Pw = sP + wave * NP, *Mw = sM + wave * NP;                 // interface values
+    const int lw = wave / WPL;   // the line this wave reconstructs
+    double *Pw = sP + lw * NP, *Mw = sM + lw * NP;                 // interface values
     double *Pd = sP + ll * NP, *Md = sM + ll * NP;
-    const bool wv = FULL || blk * LPB + wave < nll;
-    // the zones of the line this wave reconstructs (line `wave` of the
+    const bool wv = FULL || blk * LPB + lw < nll;
+    // the zones of the line this wave reconstructs (line `lw` of the
     // workgroup; in the y/z sweeps not the line of the thread's own cells)
-    const int offw = SEG ? (int)((blk * LPB + wave) % A.nseg) * n : 0;
+    const int offw = SEG ? (int)((blk * LPB + lw) % A.nseg) * n : 0;
     const Zone z{SEG ? n + 1 : n, A.nloc, A.ts, offw};
-    // line-buffer slots of the thread's cells c = g + 64k and of c + 1 (f^+
-    // skewed, f^- mirrored).  When R divides 64 they are affine in k (the
-    // pads between cells 64 apart are 64/R), so every access is one base
+    // line-buffer slots of the thread's cells c = g + GS k and of c + 1 (f^+
+    // skewed, f^- mirrored).  When R divides GS they are affine in k (the
+    // pads between cells GS apart are GS/R), so every access is one base
     // register plus an immediate offset instead of one address register per
     // cell held across the variable loop.
-    constexpr bool AFF = (64 % R) == 0;
-    constexpr int KS = AFF ? 64 + 64 / R : 0;
-    const int sa0 = Skew<R>::at(g), sa1 = Skew<R>::at(g + 1), sm0 = Skew<R>::mir(g), sm1 = Skew<R>::mir(g + 1);
-    auto slotP = [&](int k) { return AFF ? sa0 + KS * k : Skew<R>::at(g + 64 * k); };
-    auto slotP1 = [&](int k) { return AFF ? sa1 + KS * k : Skew<R>::at(g + 64 * k + 1); };
-    auto slotM = [&](int k) { return AFF ? sm0 - KS * k : Skew<R>::mir(g + 64 * k); };
-    auto slotM1 = [&](int k) { return AFF ? sm1 - KS * k : Skew<R>::mir(g + 64 * k + 1); };
+    constexpr bool AFF = (GS % R) == 0;
+    constexpr int KS = AFF ? GS + GS / R : 0;
+    const int sa0 = Sk::at(g), sa1 = Sk::at(g + 1), sm0 = Sk::mir(g), sm1 = Sk::mir(g + 1);
+    auto slotP = [&](int k) { return AFF ? sa0 + KS * k : Sk::at(g + GS * k); };
+    auto slotP1 = [&](int k) { return AFF ? sa1 + KS * k : Sk::at(g + GS * k + 1); };
+    auto slotM = [&](int k) { return AFF ? sm0 - KS * k : Sk::mir(g + GS * k); };
+    auto slotM1 = [&](int k) { return AFF ? sm1 - KS * k : Sk::mir(g + GS * k + 1); };
     // compute-mapping geometry of this lane (nuc_lines.h)
-    const int h = lane & 31;
-    const bool neg = lane >= 32;
-    const int chunk = neg ? 31 - h : h;
+    const int h = lane % NL;
+    const bool neg = WPL == 1 ? lane >= 32 : (bool)__builtin_amdgcn_readfirstlane(wave & 1);
+    const int chunk = neg ? NL - 1 - h : h;
     const int m0 = chunk * R;
-    const T *Lw = reinterpret_cast<const T *>((neg ? sM : sP) + wave * NP) + h * (R + 1);
+    const T *Lw = reinterpret_cast<const T *>((neg ? Mw : Pw)) + h * (R + 1);
     const int m0r = neg ? m0 + R - 1 : m0;
     const int mstep = neg ? -1 : 1;
     double res = 0.0;
@@ -345,7 +351,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     auto fetch = [&](int v, double qo[CPL], T xo[CPL]) {
 #pragma unroll
         for (int k = 0; k < CPL; k++) {
-            int c = g + 64 * k;
+            int c = g + GS * k;
             qo[k] = 0.0;
             xo[k] = T(0);
             if ((FULL || (lv && c < n)) && v < 5) {
@@ -374,7 +380,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     for (int v = 0; v < 5; v++) {
 #pragma unroll
         for (int k = 0; k < CPL; k++) {
-            int c = g + 64 * k;
+            int c = g + GS * k;
             if (FULL || (lv && c < n)) {
                 T fp, fm;
                 T spk[NSP];
@@ -391,8 +397,8 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
                 // n = 32R only the first and last cell of a thread can be near
                 // an end, so the other cells skip the copy
                 if (!SEG && (!FULL || k == 0 || k == CPL - 1)) {
-                    const int cw = (k == 0 && c < HALO) ? c + n : (c >= n - HALO ? c - n : 32 * R + HALO);
-                    Pl[Skew<R>::at(cw)] = fp; Ml[Skew<R>::mir(cw)] = fm;
+                    const int cw = (k == 0 && c < HALO) ? c + n : (c >= n - HALO ? c - n : NL * R + HALO);
+                    Pl[Sk::at(cw)] = fp; Ml[Sk::mir(cw)] = fm;
                     if (A.vis != VIS_NONE && v > 0) Vl[cw] = xv[k];
                 }
             }
@@ -401,7 +407,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
             if (hown) {
                 T fp, fm;
                 split_var<RIE, T>(sph, T(qh), v, d, fp, fm);
-                Pl[Skew<R>::at(hc)] = fp; Ml[Skew<R>::mir(hc)] = fm;
+                Pl[Sk::at(hc)] = fp; Ml[Sk::mir(hc)] = fm;
                 if (A.vis != VIS_NONE && v > 0) Vl[hc] = xh;
             }
         }
@@ -411,14 +417,14 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         double qhn = 0.0;
         T xhn = T(0);
         if constexpr (SEG) fetch_h(v + 1, qhn, xhn);
-        sync_lines(d);
+        sync_lines<WPL>(d);
         double out[R];
         // weights and rows in T where FP32 keeps them in range; the Z-type
         // weights (WENO5-Z, WENO7-Z and the hccs family) square tau/(is+eps)
         // with eps down to 1e-40 and stay FP64
         constexpr bool zw = SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78;
         using TW = typename std::conditional<zw, double, T>::type;
-        if (wv) line_half<SCH, R, T, TW, double>(Lw, m0r, mstep, z, h, neg, out, FULL);
+        if (wv) line_half<SCH, R, T, TW, double, NL>(Lw, m0r, mstep, z, h, neg, out, FULL);
         // the interface values overwrite the wave's own line only: the
         // reconstruction of the other waves is not waited for
         sync_wave();
@@ -431,16 +437,16 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
             double *Ow = Ob - (neg ? 1 : 0);
             // a segment's interfaces are 0..n, a periodic line's 0..n-1
             const int nif = SEG ? n + 1 : n;
-            if (FULL || m0r < nif) Ob[neg ? Skew<R>::at(-1) : Skew<R>::at(0)] = out[0];
+            if (FULL || m0r < nif) Ob[neg ? Sk::at(-1) : Sk::at(0)] = out[0];
 #pragma unroll
             for (int r = 1; r < R; r++) {
                 int m = m0r + mstep * r;
-                if (FULL || m < nif) Ow[Skew<R>::at(r)] = out[r];
+                if (FULL || m < nif) Ow[Sk::at(r)] = out[r];
             }
             // periodic copy of interface 0 to interface n
             if constexpr (!SEG) {
-                if (!neg && h == 0) Pw[Skew<R>::at(n)] = out[0];
-                if (neg && h == 31) Mw[Skew<R>::mir(n)] = out[R - 1];
+                if (!neg && h == 0) Pw[Sk::at(n)] = out[0];
+                if (neg && h == NL - 1) Mw[Sk::mir(n)] = out[R - 1];
             }
         }
         // the final phase's own global reads (rhs of the previous sweeps; u^n and
@@ -450,7 +456,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         double rin[CPL], unv[CPL], qcur[CPL];
 #pragma unroll
         for (int k = 0; k < CPL; k++) {
-            int c = g + 64 * k;
+            int c = g + GS * k;
             rin[k] = 0.0;
             unv[k] = 0.0;
             qcur[k] = 0.0;
@@ -461,10 +467,10 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
                 else if (epi) qcur[k] = lds(A.q[v], k);
             }
         }
-        sync_lines(d);
+        sync_lines<WPL>(d);
 #pragma unroll
         for (int k = 0; k < CPL; k++) {
-            int c = g + 64 * k;
+            int c = g + GS * k;
             if (FULL || (lv && c < n)) {
                 double r = rin[k];
                 // F = f^+ + f^- at the interfaces, then (F[i+1]-F[i])/dx (src/euler3d.cpp:23-56,132-166)
@@ -490,7 +496,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
                 }
             }
         }
-        sync_lines(d);
+        sync_lines<WPL>(d);
         // unconditional, so that the current values are dead after the load
         // phase instead of being carried to the end of the iteration
 #pragma unroll
@@ -505,16 +511,16 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         __syncthreads();
         if (t == 0) {
             double acc = 0.0;
-            for (int w = 0; w < LPB; w++) acc += sRed[w];
+            for (int w = 0; w < LPB * WPL; w++) acc += sRed[w];
             A.res_part[blk] = acc;
         }
     }
 }
 
-template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false>
-__global__ __launch_bounds__(64 * LPB) void k_sweep(SweepArgs A)
+template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1>
+__global__ __launch_bounds__(64 * LPB * WPL) void k_sweep(SweepArgs A)
 {
-    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI, S, SEG>(A, xcd_block(blockIdx.x, gridDim.x));
+    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI, S, SEG, WPL>(A, xcd_block(blockIdx.x, gridDim.x));
 }
 
 constexpr int SWEEP_LPB = 4;
@@ -534,81 +540,96 @@ constexpr bool mixed_fp32()
 
 constexpr bool compact_scheme(int sch) { return sch == CRWENO5 || sch == HCCS || sch == HCCS77; }
 
-// segments of lines longer than 512 cells: R = 8 (up to 255 cells), and for
-// the compact schemes R = 16 (one rank block of up to 511 cells)
-template <int SCH, int RIE, int R>
-void launch_sweep_seg(const SweepArgs &A, hipStream_t s)
-{
-    const long nb = (A.nlines * A.nseg + SWEEP_LPB - 1) / SWEEP_LPB;
-    const dim3 grid((unsigned)nb), block(64 * SWEEP_LPB);
-    if constexpr (mixed_fp32<SCH>()) {
-        if (A.fp32) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, float, false, EPI_ARG, float, true>), grid, block, 0, s, A);
-            return;
-        }
-        if (A.mixed) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, float, false, EPI_ARG, double, true>), grid, block, 0, s, A);
-            return;
-        }
-    }
-    hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, double, false, EPI_ARG, double, true>), grid, block, 0, s, A);
-}
+// Lines per workgroup of the two-wave form.  x: 2, so that a barrier holds 4
+// waves (512x256^2 CRWENO5 1.98 ms a sweep against 2.60 with 4 lines, 512x128^2
+// WENO5-Z/AUSM 0.40 against 0.51).  y and z: 4, whose loads read 32 contiguous
+// bytes per cell (512x64x512 WENO5-JS z 0.86 ms against 1.26 with 2), but 2 for
+// hccs and hccs77, whose 130-169 registers leave room for one workgroup of 8
+// waves on a CU (512^3 hccs/AUSM z 15.2 ms against 16.4).
+constexpr int lpb2_yz(int sch) { return sch == HCCS || sch == HCCS77 ? 2 : SWEEP_LPB; }
+constexpr int sweep_lpb(int wpl, int dir, int sch) { return wpl == 1 ? SWEEP_LPB : dir == 0 ? 2 : lpb2_yz(sch); }
 
 // the kernel forms for one state type S and stencil type T: FULL kernels
-// (n = 32R, even R) with and without the RK3 update, else the one that takes
-// it as an argument
-template <int SCH, int RIE, int R, typename T, typename S>
-void launch_sweep_rt(const SweepArgs &A, hipStream_t s, bool full, dim3 grid, dim3 block)
+// (every lane's rows on the line, even R) with and without the RK3 update,
+// else the one that takes it as an argument
+template <int SCH, int RIE, int R, int WPL, int LPB, bool SEG, typename T, typename S>
+void launch_sweep_rtl(const SweepArgs &A, hipStream_t s)
 {
-    if constexpr (R % 2 == 0) {
+    const dim3 grid((unsigned)((A.nlines * A.nseg + LPB - 1) / LPB)), block(64 * LPB * WPL);
+    // odd R: the load mapping's cells overrun the line, so no FULL form
+    if constexpr (!SEG && R % 2 == 0) {
+        const bool full = A.n == 32 * WPL * R && A.nlines % LPB == 0;
         if (full && A.epilogue) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, T, true, EPI_YES, S>), grid, block, 0, s, A);
+            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_YES, S, false, WPL>), grid, block, 0, s, A);
             return;
         }
         if (full) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, T, true, EPI_NO, S>), grid, block, 0, s, A);
+            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_NO, S, false, WPL>), grid, block, 0, s, A);
             return;
         }
     }
-    hipLaunchKernelGGL((k_sweep<SCH, RIE, R, SWEEP_LPB, T, false, EPI_ARG, S>), grid, block, 0, s, A);
+    hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, false, EPI_ARG, S, SEG, WPL>), grid, block, 0, s, A);
 }
 
-template <int SCH, int RIE, int R>
+template <int SCH, int RIE, int R, int WPL, bool SEG, typename T, typename S>
+void launch_sweep_rt(const SweepArgs &A, hipStream_t s)
+{
+    constexpr int LX = sweep_lpb(WPL, 0, SCH), LYZ = sweep_lpb(WPL, 1, SCH);
+    // FP32 stencils sweep x alone on two waves a line (segments: every direction)
+    constexpr bool X_ONLY = WPL == 2 && !SEG && sizeof(T) == 4;
+    if (X_ONLY || LX == LYZ || A.dir == 0) launch_sweep_rtl<SCH, RIE, R, WPL, LX, SEG, T, S>(A, s);
+    else if constexpr (!X_ONLY) launch_sweep_rtl<SCH, RIE, R, WPL, LYZ, SEG, T, S>(A, s);
+}
+
+template <int SCH, int RIE, int R, int WPL, bool SEG = false>
 void launch_sweep_r(const SweepArgs &A, hipStream_t s)
 {
-    if (A.nseg > 1) {
-        if constexpr (R == 8 || (R == 16 && compact_scheme(SCH))) launch_sweep_seg<SCH, RIE, R>(A, s);
-        return;
-    }
-    long nb = (A.nlines + SWEEP_LPB - 1) / SWEEP_LPB;
-    // odd R: the load mapping's 64 (R+1)/2 cells overrun a 32R-cell line, so no FULL form
-    const bool full = (R % 2 == 0) && (A.n == 32 * R) && (A.nlines % SWEEP_LPB == 0);
-    const dim3 grid((unsigned)nb), block(64 * SWEEP_LPB);
     if constexpr (mixed_fp32<SCH>()) {
         if (A.fp32) {   // NUC_FP32: FP32 state and RHS around the mixed path's arithmetic
-            launch_sweep_rt<SCH, RIE, R, float, float>(A, s, full, grid, block);
+            launch_sweep_rt<SCH, RIE, R, WPL, SEG, float, float>(A, s);
             return;
         }
         if (A.mixed) {
-            launch_sweep_rt<SCH, RIE, R, float, double>(A, s, full, grid, block);
+            launch_sweep_rt<SCH, RIE, R, WPL, SEG, float, double>(A, s);
             return;
         }
     }
-    launch_sweep_rt<SCH, RIE, R, double, double>(A, s, full, grid, block);
+    // FP64 stencils take more than 8 rows a lane on two waves only
+    if constexpr (R <= 8) launch_sweep_rt<SCH, RIE, R, WPL, SEG, double, double>(A, s);
 }
 
+// rows per lane and waves per line: the forms sweep_rows / sweep_wpl
+// (nuc3d.hip) choose from
 template <int SCH, int RIE>
 void launch_sweep_sr(int R, const SweepArgs &A, hipStream_t s)
 {
+    if (A.nseg > 1) {   // lines longer than 512 cells; whole blocks of 256-511 cells only with the compact schemes
+        if constexpr (compact_scheme(SCH))
+            if (A.wpl == 2) { launch_sweep_r<SCH, RIE, 8, 2, true>(A, s); return; }
+        launch_sweep_r<SCH, RIE, 8, 1, true>(A, s);
+        return;
+    }
+    if (A.wpl == 2) {
+        switch (R) {
+        case 5: launch_sweep_r<SCH, RIE, 5, 2>(A, s); break;
+        case 6: launch_sweep_r<SCH, RIE, 6, 2>(A, s); break;
+        default: launch_sweep_r<SCH, RIE, 8, 2>(A, s); break;
+        }
+        return;
+    }
     switch (R) {
-    case 2: launch_sweep_r<SCH, RIE, 2>(A, s); break;
-    case 3: launch_sweep_r<SCH, RIE, 3>(A, s); break;
-    case 4: launch_sweep_r<SCH, RIE, 4>(A, s); break;
-    case 5: launch_sweep_r<SCH, RIE, 5>(A, s); break;
-    case 6: launch_sweep_r<SCH, RIE, 6>(A, s); break;
-    case 8: launch_sweep_r<SCH, RIE, 8>(A, s); break;
-    case 12: launch_sweep_r<SCH, RIE, 12>(A, s); break;
-    default: launch_sweep_r<SCH, RIE, 16>(A, s); break;
+    case 2: launch_sweep_r<SCH, RIE, 2, 1>(A, s); break;
+    case 3: launch_sweep_r<SCH, RIE, 3, 1>(A, s); break;
+    case 4: launch_sweep_r<SCH, RIE, 4, 1>(A, s); break;
+    case 5: launch_sweep_r<SCH, RIE, 5, 1>(A, s); break;
+    case 6: launch_sweep_r<SCH, RIE, 6, 1>(A, s); break;
+    case 8: launch_sweep_r<SCH, RIE, 8, 1>(A, s); break;
+    default:
+        if constexpr (mixed_fp32<SCH>()) {
+            if (R == 12) launch_sweep_r<SCH, RIE, 12, 1>(A, s);
+            else launch_sweep_r<SCH, RIE, 16, 1>(A, s);
+        }
+        break;
     }
 }
 

@@ -22,6 +22,18 @@ CASES = [
     # one WENO7-Z evaluation for both kinds of row
     ((10, 20, 30), (1, 2, 3), G.HCCS77, G.CD6, G.AUSM),
     ((10, 20, 30), (1, 2, 3), G.HCCS78, G.CD8, G.LF),
+    # two waves per line (257-512 cells): one cell more than a wave holds, the
+    # ends of each row count, tails of the lines per workgroup (2 in x, 4 or 2
+    # in y and z), a compact segment of 511 cells
+    ((257, 11, 12), (1, 1, 1), G.CRWENO5, G.CD8, G.LF),
+    ((11, 320, 13), (1, 1, 1), G.HCCS, G.CD6, G.AUSM),
+    ((13, 11, 321), (1, 1, 1), G.WENO5Z, G.CD6, G.AUSM),
+    ((384, 12, 10), (2, 1, 1), G.HCCS77, G.CD6, G.LF),
+    ((11, 385, 10), (1, 1, 1), G.WENO7JS, G.CD8, G.AUSMP),
+    ((10, 511, 11), (1, 1, 1), G.CRWENO5, G.CD6, G.AUSM),
+    ((512, 10, 11), (1, 1, 1), G.HCCS, G.CD6, G.LF),
+    ((12, 10, 512), (1, 1, 4), G.CRWENO5, G.CD8, G.LF),
+    ((1022, 10, 11), (2, 1, 1), G.CRWENO5, G.CD6, G.LF),
 ]
 
 
