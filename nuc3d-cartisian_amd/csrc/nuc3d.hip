@@ -982,7 +982,7 @@ extern "C" int nuc_create(const nuc_config *cfg, nuc_ctx **out)
     // residual partials: one per workgroup of the last sweep
     const int dl = kSweepOrder[2];
     long lines_last = x->N / x->n[dl] * x->nseg[dl];
-    const int lpb_last = sweep_lpb(x->wpl[dl], dl, cfg->scheme[dl]);
+    const int lpb_last = sweep_lpb(x->wpl[dl], dl, cfg->scheme[dl], cfg->riemann);
     x->res_nb = (lines_last + lpb_last - 1) / lpb_last;
     if (!dalloc(&x->res_part, x->res_nb * sizeof(double))) return fail("device allocation (residual)");
     (void)hipMemsetAsync(x->lam, 0, 3 * MAXRANK * sizeof(unsigned long long), x->stream);

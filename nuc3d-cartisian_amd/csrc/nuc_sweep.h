@@ -191,6 +191,46 @@ __device__ __forceinline__ void sync_lines(int d)
     else __syncthreads();
 }
 
+// Where a sweep kernel keeps what, and the waves per SIMD it is built for
+// (WAVES: at most 512/WAVES registers and 160 KB/(4 WAVES) of LDS a wave;
+// 1: whatever the compiler takes).
+// A wave of the sweep spends most of its time waiting (LDS round trips, the
+// serial parts of the solve, barriers, its final loads), so the number of waves
+// decides: FP64 CRWENO5/LF at R = 8 took 53 KB and 129-137 registers, three
+// waves, with its three split parameters in LDS and the next variable's loads
+// held across the reconstruction.  One parameter in LDS, two in registers and
+// those loads issued after the reconstruction make 37 KB and 123-128 registers,
+// four waves: 256^3 x 0.89 -> 0.81 ms, y 0.95 -> 0.90, z 0.93 -> 0.89.  The
+// AUSM form (five parameters, three in LDS) goes from two waves to three: x 1.06
+// -> 0.91, y 1.07 -> 0.97, z 1.02 -> 0.95; hccs/AUSM x 1.34 -> 1.13, y 1.37 ->
+// 1.19, z 1.32 -> 1.16.  The explicit schemes with AUSM move up to three of
+// their five parameters to LDS for a fourth wave (WENO5-Z 256^3 x 0.73 -> 0.67,
+// WENO7 160^3 x 0.354 -> 0.337).  Their 8-row form with tails needs 159
+// registers and stays at three waves (230^3 0.72 ms against 0.75 with one
+// parameter in LDS).
+template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct SweepForm {
+    static constexpr bool COMPACT = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
+    static constexpr int NL = 32 * WPL;           // lanes per sign
+    static constexpr int GS = 64 * WPL;           // threads per line in the load mapping
+    static constexpr int CPL = (R + 1) / 2;       // cells per thread in the load mapping (odd R: the last slot of
+                                                  // the upper half of the threads is past the line)
+    static constexpr int NSP = RIE == RIE_LF ? 3 : 5;
+    static constexpr int NP = Skew<R, NL>::pitch(NL * R);
+    static constexpr int NV = plain_pitch(NL * R);
+    static constexpr bool D64 = sizeof(T) == 8, LF = RIE == RIE_LF;
+    static constexpr bool FREE = R < 5 || R >= 12 || (!COMPACT && D64 && !LF && R == 8 && EPI == EPI_ARG);
+    static constexpr int WAVES = FREE ? 1 : COMPACT && D64 && (SCH != CRWENO5 || !LF) ? 3 : 4;
+    static constexpr int LDS = 163840 * LPB * WPL / (4 * WAVES) - 64;           // bytes of a workgroup
+    static constexpr int LINES = LPB * (2 * NP * (int)sizeof(double) + NV * (int)sizeof(T));
+    static constexpr int SPB = CPL * GS * LPB * (int)sizeof(T);               // one split parameter of every cell
+    static constexpr int FIT = (LDS - LINES) / SPB < 0 ? 0 : (LDS - LINES) / SPB;
+    static constexpr int WANT = COMPACT ? NSP : LF ? 0 : 3;
+    // split parameters of a cell kept in LDS, the others in registers
+    static constexpr int NLD = FREE ? (COMPACT ? NSP : 0) : FIT < WANT ? FIT : WANT;
+    // whether the next variable's global loads are held across the reconstruction
+    static constexpr bool PREF = !(D64 && R == 8 && WAVES == 4 && (COMPACT || !LF));
+};
+
 // T: type of the split fluxes, line buffers and stencils (double, or float
 // for the mixed path); weights, tridiagonal solves, interface values, the
 // flux difference and the RHS/RK3 accumulation are FP64 in both.
@@ -209,14 +249,9 @@ template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, type
 __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
 {
     const bool epi = EPI == EPI_ARG ? A.epilogue != 0 : EPI == EPI_YES;
-    constexpr int NL = 32 * WPL;           // lanes per sign
+    using F = SweepForm<SCH, RIE, R, LPB, T, EPI, WPL>;
+    constexpr int NL = F::NL, GS = F::GS, CPL = F::CPL, NSP = F::NSP, NP = F::NP, NV = F::NV, NLD = F::NLD;
     using Sk = Skew<R, NL>;
-    constexpr int GS = 64 * WPL;           // threads per line in the load mapping
-    constexpr int NP = Sk::pitch(NL * R);
-    constexpr int NV = plain_pitch(NL * R);
-    constexpr int CPL = (R + 1) / 2;       // cells per thread in the load mapping (odd R: the last slot of
-                                           // the upper half-wave is past the line)
-    constexpr int NSP = (RIE == RIE_LF) ? 3 : 5;
     constexpr int RAD = Radius<SCH>::value;
     // sP/sM hold the split fluxes (as T) and then the interface values (as
     // double) of the same lines; the phases are separated by barriers
@@ -261,14 +296,11 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         return double(ld_at(static_cast<const S GMEM *>(p), o >> SSH, fb >> SSH));
     };
 
-    // split parameters of the own cells (con2prim, src/physicsModel.cpp:331-344).
-    // The compact schemes keep them in LDS (one column per thread, read back
-    // by the same thread): their chunk solve needs the registers.  The
-    // explicit schemes keep them in CPL*NSP registers: with the LDS copy the
-    // workgroup's 53 KB (LF) would allow only three workgroups per CU.
-    constexpr bool SP_LDS = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
-    __shared__ T sSP[SP_LDS ? CPL * NSP : 1][SP_LDS ? GS * LPB : 1];
-    T spr[SP_LDS ? 1 : CPL][SP_LDS ? 1 : NSP];
+    // split parameters of the own cells (con2prim, src/physicsModel.cpp:331-344):
+    // the first NLD in LDS (one column per thread, read back by the same
+    // thread), the others in registers
+    __shared__ T sSP[NLD > 0 ? CPL * NLD : 1][NLD > 0 ? GS * LPB : 1];
+    T spr[CPL][NSP];
     unsigned innermask = 0;   // cd8 inner-form cells (rank-local position)
 #pragma unroll
     for (int k = 0; k < CPL; k++) {
@@ -281,7 +313,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         split_params<RIE, T>(q, d, T(A.gamma), tmp, A.riemann == RIE_AUSMP);
 #pragma unroll
         for (int j = 0; j < NSP; j++) {
-            if constexpr (SP_LDS) sSP[k * NSP + j][t] = tmp[j];
+            if (j < NLD) sSP[k * NLD + j][t] = tmp[j];
             else spr[k][j] = tmp[j];
         }
         int cl = (c + off) % A.nloc;
@@ -386,7 +418,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
                 T spk[NSP];
 #pragma unroll
                 for (int j = 0; j < NSP; j++) {
-                    if constexpr (SP_LDS) spk[j] = sSP[k * NSP + j][t];
+                    if (j < NLD) spk[j] = sSP[k * NLD + j][t];
                     else spk[j] = spr[k][j];
                 }
                 split_var<RIE, T>(spk, T(qv[k]), v, d, fp, fm);
@@ -413,7 +445,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         }
         double qnx[CPL];
         T xnx[CPL];
-        fetch(v + 1, qnx, xnx);   // v + 1 = 5 gives zeros
+        if constexpr (F::PREF) fetch(v + 1, qnx, xnx);   // v + 1 = 5 gives zeros
         double qhn = 0.0;
         T xhn = T(0);
         if constexpr (SEG) fetch_h(v + 1, qhn, xhn);
@@ -449,6 +481,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
                 if (neg && h == NL - 1) Mw[Sk::mir(n)] = out[R - 1];
             }
         }
+        if constexpr (!F::PREF) fetch(v + 1, qnx, xnx);
         // the final phase's own global reads (rhs of the previous sweeps; u^n and
         // the current state of the RK update), issued after the reconstruction:
         // held across it they would cost 3*CPL registers, and the other waves
@@ -518,7 +551,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
 }
 
 template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1>
-__global__ __launch_bounds__(64 * LPB * WPL) void k_sweep(SweepArgs A)
+__global__ __launch_bounds__(64 * LPB * WPL, (SweepForm<SCH, RIE, R, LPB, T, EPI, WPL>::WAVES)) void k_sweep(SweepArgs A)
 {
     sweep_body<SCH, RIE, R, LPB, T, FULL, EPI, S, SEG, WPL>(A, xcd_block(blockIdx.x, gridDim.x));
 }
@@ -546,8 +579,8 @@ constexpr bool compact_scheme(int sch) { return sch == CRWENO5 || sch == HCCS ||
 // bytes per cell (512x64x512 WENO5-JS z 0.86 ms against 1.26 with 2), but 2 for
 // hccs and hccs77, whose 130-169 registers leave room for one workgroup of 8
 // waves on a CU (512^3 hccs/AUSM z 15.2 ms against 16.4).
-constexpr int lpb2_yz(int sch) { return sch == HCCS || sch == HCCS77 ? 2 : SWEEP_LPB; }
-constexpr int sweep_lpb(int wpl, int dir, int sch) { return wpl == 1 ? SWEEP_LPB : dir == 0 ? 2 : lpb2_yz(sch); }
+constexpr int lpb2_yz(int sch, int rie) { return sch == HCCS || sch == HCCS77 || (sch == CRWENO5 && rie != RIE_LF) ? 2 : SWEEP_LPB; }
+constexpr int sweep_lpb(int wpl, int dir, int sch, int rie) { return wpl == 1 ? SWEEP_LPB : dir == 0 ? 2 : lpb2_yz(sch, rie); }
 
 // the kernel forms for one state type S and stencil type T: FULL kernels
 // (every lane's rows on the line, even R) with and without the RK3 update,
@@ -574,7 +607,7 @@ void launch_sweep_rtl(const SweepArgs &A, hipStream_t s)
 template <int SCH, int RIE, int R, int WPL, bool SEG, typename T, typename S>
 void launch_sweep_rt(const SweepArgs &A, hipStream_t s)
 {
-    constexpr int LX = sweep_lpb(WPL, 0, SCH), LYZ = sweep_lpb(WPL, 1, SCH);
+    constexpr int LX = sweep_lpb(WPL, 0, SCH, RIE), LYZ = sweep_lpb(WPL, 1, SCH, RIE);
     // FP32 stencils sweep x alone on two waves a line (segments: every direction)
     constexpr bool X_ONLY = WPL == 2 && !SEG && sizeof(T) == 4;
     if (X_ONLY || LX == LYZ || A.dir == 0) launch_sweep_rtl<SCH, RIE, R, WPL, LX, SEG, T, S>(A, s);
