@@ -21,6 +21,7 @@
 #include "nuc_lines.h"
 #include "nuc_sweep.h"
 #include "nuc_force.h"
+#include "nuc_transfer.h"
 #include "../host/hit_spectrum.hpp"
 
 #include <hip/hip_runtime.h>
@@ -948,6 +949,7 @@ extern "C" int nuc_create(const nuc_config *cfg, nuc_ctx **out)
         delete x;
         return NUC_EHIP;
     }
+    nuctransfer::retain();
     auto dalloc = [&](auto **ptr, size_t bytes) {
         return hipMallocAsync(reinterpret_cast<void **>(ptr), bytes, x->stream) == hipSuccess;
     };
@@ -997,6 +999,7 @@ extern "C" int nuc_destroy(nuc_ctx *x)
     if (!x) return NUC_OK;
     if (!x->stream) { delete x; return NUC_OK; }
     (void)hipStreamSynchronize(x->stream);
+    nuctransfer::release();
     if (x->gexec) (void)hipGraphExecDestroy(x->gexec);
     if (x->graph) (void)hipGraphDestroy(x->graph);
     void *bufs[] = {x->q[0], x->q[1], x->q[2], x->rhs, x->prim, x->fv, x->lam, x->scal, x->res_part,
@@ -1064,7 +1067,7 @@ extern "C" int nuc_upload_state(nuc_ctx *x, const double *q)
 {
     if (!x || !q) return NUC_EINVAL;
     x->next_stage = 0;   // an upload starts a new step
-    NUC_CHECK(x, hipMemcpyAsync(state64_w(x), q, 5 * x->N * sizeof(double), hipMemcpyHostToDevice, x->stream));
+    NUC_CHECK(x, nuctransfer::copy(state64_w(x), q, 5 * x->N * sizeof(double), hipMemcpyHostToDevice, x->stream));
     state64_commit(x);
     NUC_CHECK(x, hipStreamSynchronize(x->stream));
     return NUC_OK;
@@ -1073,8 +1076,7 @@ extern "C" int nuc_upload_state(nuc_ctx *x, const double *q)
 extern "C" int nuc_download_state(nuc_ctx *x, double *q)
 {
     if (!x || !q) return NUC_EINVAL;
-    NUC_CHECK(x, hipMemcpyAsync(q, state64(x), 5 * x->N * sizeof(double), hipMemcpyDeviceToHost, x->stream));
-    NUC_CHECK(x, hipStreamSynchronize(x->stream));
+    NUC_CHECK(x, nuctransfer::copy(q, state64(x), 5 * x->N * sizeof(double), hipMemcpyDeviceToHost, x->stream));
     return NUC_OK;
 }
 
@@ -1512,7 +1514,7 @@ extern "C" int nuc_rhs(nuc_ctx *x, double *rhs_host, double *dt_local)
                                reinterpret_cast<const float *>(x->rhs), x->q64, 5 * x->N);
             r = x->q64;
         }
-        NUC_CHECK(x, hipMemcpyAsync(rhs_host, r, 5 * x->N * sizeof(double), hipMemcpyDeviceToHost, x->stream));
+        NUC_CHECK(x, nuctransfer::copy(rhs_host, r, 5 * x->N * sizeof(double), hipMemcpyDeviceToHost, x->stream));
     }
     double sc[8];
     NUC_CHECK(x, hipMemcpyAsync(sc, x->scal, sizeof(sc), hipMemcpyDeviceToHost, x->stream));
@@ -2215,8 +2217,8 @@ extern "C" int nuc_average_restore(nuc_ctx *x, int type, long long steps, const 
     size_t off = 0;
     for (int g = 0; g < ng; g++) {
         const size_t n = (size_t)cnt[g] * x->N;
-        NUC_CHECK(x, hipMemcpyAsync(x->post_buf + seg[g], fields + off, n * sizeof(double), hipMemcpyHostToDevice,
-                                    x->stream));
+        NUC_CHECK(x, nuctransfer::copy(x->post_buf + seg[g], fields + off, n * sizeof(double), hipMemcpyHostToDevice,
+                                       x->stream));
         off += n;
     }
     NUC_CHECK(x, hipStreamSynchronize(x->stream));
@@ -2244,9 +2246,8 @@ extern "C" int nuc_average_field(nuc_ctx *x, int group, int index, double *out)
         x->err = "no such averaged field at this averaging type";
         return NUC_EINVAL;
     }
-    NUC_CHECK(x, hipMemcpyAsync(out, x->post_buf + seg + (long)index * x->N, x->N * sizeof(double),
-                                hipMemcpyDeviceToHost, x->stream));
-    NUC_CHECK(x, hipStreamSynchronize(x->stream));
+    NUC_CHECK(x, nuctransfer::copy(out, x->post_buf + seg + (long)index * x->N, x->N * sizeof(double),
+                                   hipMemcpyDeviceToHost, x->stream));
     return NUC_OK;
 }
 
@@ -2727,7 +2728,7 @@ extern "C" int nuc_q_fields(nuc_ctx *x, double *out)
     QArgs Q{gp(q64), gp((const double *)uvw), gp(f), N};
     hipLaunchKernelGGL(k_qfields, grid, blk, 0, x->stream, Q);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(out, f, 16 * (size_t)N * sizeof(double), hipMemcpyDeviceToHost, x->stream);
+    if (e == hipSuccess) e = nuctransfer::copy(out, f, 16 * (size_t)N * sizeof(double), hipMemcpyDeviceToHost, x->stream);
     (void)hipFreeAsync(buf, x->stream);
     hipError_t e2 = hipStreamSynchronize(x->stream);
     if (e != hipSuccess || e2 != hipSuccess) {
