@@ -10,7 +10,8 @@ namespace nuctransfer {
 // hipMemcpyAsync takes is accepted.
 hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s);
 
-// The staging memory is kept while contexts exist: every context holds it once.
+// The staging memory is kept while someone holds it: every context and every
+// serving loop (whose contexts come and go) does, once.
 void retain();
 void release();
 

@@ -33,6 +33,7 @@ constexpr size_t MIN_UP = size_t(16) << 20, MIN_DOWN = size_t(8) << 20;
 std::mutex g_mu;                       // the staging memory and its user count
 char *g_stage = nullptr;               // 2 * THREADS slots of CHUNK bytes (64 MiB), pinned
 int g_users = 0;
+size_t g_seen = 0;                     // bytes that would have been staged since the memory was last given back
 
 // A chunk into a pinned slot by stores over the link.  hipMemcpyAsync down
 // followed by an event costs 130 us a copy here whatever its size (4 MiB
@@ -112,7 +113,10 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
         // one staged copy at a time; another thread's takes the plain path meanwhile
         std::unique_lock<std::mutex> lk(g_mu, std::try_to_lock);
         if (lk.owns_lock()) {
-            if (!g_stage && hipHostMalloc((void **)&g_stage, 2 * THREADS * CHUNK, hipHostMallocPortable) != hipSuccess) {
+            // pinning it takes about 4 ms: only once the arrays have made up for that
+            g_seen += bytes;
+            if (!g_stage && g_seen >= 2 * THREADS * CHUNK &&
+                hipHostMalloc((void **)&g_stage, 2 * THREADS * CHUNK, hipHostMallocPortable) != hipSuccess) {
                 g_stage = nullptr;
                 (void)hipGetLastError();
             }
@@ -150,9 +154,10 @@ void retain()
 void release()
 {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (--g_users == 0 && g_stage) {
-        (void)hipHostFree(g_stage);
+    if (--g_users == 0) {
+        if (g_stage) (void)hipHostFree(g_stage);
         g_stage = nullptr;
+        g_seen = 0;
     }
 }
 

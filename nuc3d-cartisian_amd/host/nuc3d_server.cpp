@@ -315,12 +315,19 @@ void nuc_server::launch_idle(std::vector<std::shared_ptr<Job>> &idle)
     }
 }
 
+// csrc/nuc_transfer.h, which needs the HIP headers
+namespace nuctransfer {
+void retain();
+void release();
+}
+
 extern "C" int nuc_server_create(const nuc_server_config *cfg, nuc_server **out)
 {
     if (!cfg || !out || cfg->max_active < 1 || cfg->hbm_budget <= 0) return NUC_EINVAL;
     nuc_server *s = new nuc_server();
     s->cfg = *cfg;
     s->worker = std::thread([s] { s->run(); });
+    nuctransfer::retain();
     *out = s;
     return NUC_OK;
 }
@@ -338,6 +345,7 @@ extern "C" int nuc_server_destroy(nuc_server *s)
     s->packs.clear();
     for (auto &j : s->active)
         if (j->ctx) nuc_destroy(j->ctx);
+    nuctransfer::release();
     delete s;
     return NUC_OK;
 }
