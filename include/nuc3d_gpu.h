@@ -152,7 +152,8 @@ int nuc_set_graph(nuc_ctx *ctx, int enable);
  * fastest; the choice is cached per (nx, ny, nz, precision) for the process.
  * Results do not depend on the tile shape.  No counterpart in the reference.
  * nuc_tile_shape reports the shape in use; nuc_set_tile_shape sets it
- * (1 <= planes <= nz). */
+ * (1 <= planes <= nz).  On boxes too small to fill the GPU with it the kernel
+ * cuts its marches shorter than the shape says. */
 int nuc_autotune(nuc_ctx *ctx);
 int nuc_tile_shape(const nuc_ctx *ctx, int *grad_planes);
 int nuc_set_tile_shape(nuc_ctx *ctx, int grad_planes);

@@ -169,6 +169,7 @@ struct DtArgs {
     int P, set_global;
     double hx, hy, hz, cfl;
     double GMEM *scal;
+    double GMEM *dt_out;      // nuc_rhs_noalloc: the caller's dt, or null
 };
 
 __device__ __forceinline__ void dt_body(const DtArgs &A)
@@ -184,11 +185,15 @@ __device__ __forceinline__ void dt_body(const DtArgs &A)
         }
         A.scal[3] = dtmin;
         if (A.set_global) A.scal[0] = dtmin * A.cfl;
+        if (A.dt_out) *A.dt_out = dtmin;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 3 * A.P; i += blockDim.x) A.lam[i] = 0ull;
 }
 
+// A launch of its own: taken by k_prim's last workgroup instead, dt costs a
+// release of every workgroup's maxima to the other XCDs, and a 97x60x83
+// right-hand side goes from 186 to 197 us, a 64^3 step from 185 to 196.
 __global__ void k_dt(DtArgs A) { dt_body(A); }
 
 // ---------------------------------------------------------------------------
@@ -205,9 +210,31 @@ __device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >
 // neighbouring workgroups), instead of the 27 stencil reads per field of a
 // gather kernel, and no primitive field round-trips through HBM.
 constexpr int GTX = 32, GTY = 16;
-// planes per workgroup: long marches amortise the 8-plane z halo on large
-// boxes; short ones give small boxes enough workgroups
-inline int grad_planes(int nz) { return nz >= 256 ? 32 : (nz >= 128 ? 16 : (nz >= 64 ? 8 : 4)); }
+// Planes per workgroup of the march: a workgroup costs its planes and about two
+// more for the queue's first eight, and one FP64 workgroup fills a CU, so the
+// march takes as many rounds of the 256 CUs as it has workgroups.  The least
+// rounds x (planes + 2), and of equals the longer march (fewer halo planes).
+// Measured (FP64, us, by planes 1 2 4 8 16 32): 32^3 6 9 15 27 - -; 64^3 16 12 16
+// 28 52 -; 96^3 62 55 41 34 54 -; 128^3 133 100 82 74 69 112; 256^3 1167 903 727
+// 639 599 581.
+inline int march_planes(int nx, int ny, int nz, int most)
+{
+    const long tiles = (long)((nx + GTX - 1) / GTX) * ((ny + GTY - 1) / GTY);
+    long best = 0;
+    int planes = 1;
+    for (int g = most; g >= 1; g = g > 32 ? 32 : g & (g - 1) ? g & (g - 1) : g / 2) {
+        const long rounds = (tiles * ((nz + g - 1) / g) + 255) / 256, cost = rounds * (g + 2);
+        if (best == 0 || cost < best) { best = cost; planes = g; }
+    }
+    return planes;
+}
+inline int grad_planes(int nx, int ny, int nz) { return march_planes(nx, ny, nz, nz < 32 ? nz : 32); }
+// the march of a tile shape of g planes: cut where it would leave CUs idle
+inline int cut_planes(int nx, int ny, int nz, int g)
+{
+    const long tiles = (long)((nx + GTX - 1) / GTX) * ((ny + GTY - 1) / GTY);
+    return tiles * ((nz + g - 1) / g) >= 256 ? g : march_planes(nx, ny, nz, g);
+}
 
 // primitives u, v, w, T of one cell from its five conserved values
 // (src/physicsModel.cpp:331-344, the same expression as k_prim)
@@ -374,9 +401,14 @@ __device__ __forceinline__ void res_body(const ResArgs &A)
     double GMEM *scal = A.scal;
     const double inv_count = A.inv_count;
     __shared__ double sm[256];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < nb; i += 256) acc += part[i];
-    sm[threadIdx.x] = acc;
+    // one workgroup over all partials: eight loads in flight a thread
+    // (256^3, 16384 partials: 24 -> 8 us)
+    double a8[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < nb; i += 8 * 256) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) a8[k] += i + 256 * k < nb ? part[i + 256 * k] : 0.0;
+    }
+    sm[threadIdx.x] = ((a8[0] + a8[1]) + (a8[2] + a8[3])) + ((a8[4] + a8[5]) + (a8[6] + a8[7]));
     __syncthreads();
     for (int s = 128; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
@@ -707,6 +739,7 @@ struct nuc_ctx {
     double *rhs = nullptr, *prim = nullptr, *fv = nullptr;
     unsigned long long *lam = nullptr;
     double *scal = nullptr;
+    double *dt_out = nullptr;            // nuc_rhs_noalloc: the caller's device slot for dt
     double *res_part = nullptr;
     long res_nb = 0;
     double *stat_part = nullptr;
@@ -1116,9 +1149,11 @@ static void stage_args(nuc_ctx *x, int in, int stage, int outb, bool epilogue, S
         P.riemann = c.riemann; P.do_lam = lam_needed ? 1 : 0; P.write_prim = wp ? 1 : 0;
         P.gamma = c.gamma; P.mach = c.mach; P.lam = gp(x->lam);
         sa.do_prim = P.do_lam || P.write_prim;
-        sa.prim_nb = std::min<long>((N + 4095) / 4096, 65536);
+        // 16 cells a thread, but two where that leaves CUs idle (64^3: 64
+        // workgroups of 16 serial loads, 8 us)
+        sa.prim_nb = std::min<long>(std::max<long>((N + 4095) / 4096, std::min<long>((N + 511) / 512, 256)), 65536);
         sa.do_dt = lam_needed;
-        sa.dt = DtArgs{gp(x->lam), x->P, epilogue ? 1 : 0, x->h[0], x->h[1], x->h[2], c.cfl, gp(x->scal)};
+        sa.dt = DtArgs{gp(x->lam), x->P, epilogue ? 1 : 0, x->h[0], x->h[1], x->h[2], c.cfl, gp(x->scal), gp(x->dt_out)};
     }
     if (ns) {
         GradArgs &G = sa.grad;
@@ -1132,7 +1167,7 @@ static void stage_args(nuc_ctx *x, int in, int stage, int outb, bool epilogue, S
         }
         G.law = c.viscosity; G.re = c.reynolds; G.mach = c.mach; G.pr = c.prandtl; G.gamma = c.gamma;
         G.tref = c.t_ref; G.tinf = c.t_inf;
-        G.gkz = x->gkz > 0 ? x->gkz : grad_planes(x->n[2]);
+        G.gkz = x->gkz > 0 ? cut_planes(x->n[0], x->n[1], x->n[2], x->gkz) : grad_planes(x->n[0], x->n[1], x->n[2]);
         sa.ggrid = dim3((x->n[0] + GTX - 1) / GTX, (x->n[1] + GTY - 1) / GTY, (x->n[2] + G.gkz - 1) / G.gkz);
         sa.do_grad = true;
     }
@@ -1355,14 +1390,13 @@ extern "C" int nuc_autotune(nuc_ctx *x)
     hipEvent_t e0, e1;
     NUC_CHECK(x, hipEventCreate(&e0));
     NUC_CHECK(x, hipEventCreate(&e1));
-    const int cand[4] = {4, 8, 16, 32};
-    int best = grad_planes(x->n[2]);
+    int best = grad_planes(x->n[0], x->n[1], x->n[2]);
     float best_ms = 1e30f;
-    for (int gkz : cand) {
+    for (int gkz : {4, 8, 16, 32}) {
         if (gkz > x->n[2]) continue;
         GradArgs G = sa.grad;
-        G.gkz = gkz;
-        const dim3 grid(sa.ggrid.x, sa.ggrid.y, (x->n[2] + gkz - 1) / gkz);
+        G.gkz = cut_planes(x->n[0], x->n[1], x->n[2], gkz);
+        const dim3 grid(sa.ggrid.x, sa.ggrid.y, (x->n[2] + G.gkz - 1) / G.gkz);
         float tot = 0.f;
         for (int rep = 0; rep < 4; rep++) {
             (void)hipEventRecord(e0, x->stream);
@@ -1399,7 +1433,7 @@ extern "C" int nuc_set_tile_shape(nuc_ctx *x, int planes)
 extern "C" int nuc_tile_shape(const nuc_ctx *x, int *grad_planes_out)
 {
     if (!x || !grad_planes_out) return NUC_EINVAL;
-    *grad_planes_out = x->gkz > 0 ? x->gkz : grad_planes(x->n[2]);
+    *grad_planes_out = x->gkz > 0 ? x->gkz : grad_planes(x->n[0], x->n[1], x->n[2]);
     return NUC_OK;
 }
 
@@ -1544,8 +1578,6 @@ __global__ void k_clear_u64(unsigned long long *p, int n)
     for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0ull;
 }
 
-__global__ void k_copy_dt(const double *scal, double *dt_out) { *dt_out = scal[3]; }
-
 extern "C" int nuc_rhs_noalloc(const nuc_config *cfg, const double *q_dev, double *rhs_dev, double *dt_local_dev,
                                void *stream)
 {
@@ -1596,6 +1628,7 @@ extern "C" int nuc_rhs_noalloc(const nuc_config *cfg, const double *q_dev, doubl
     x.fv = base;
     x.lam = reinterpret_cast<unsigned long long *>(base + NOALLOC_FV);
     x.scal = base + NOALLOC_FV + NOALLOC_LAM;
+    x.dt_out = dt_local_dev;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune_gkz.find(std::make_tuple(x.n[0], x.n[1], x.n[2], (int)cfg->precision * 2 + (x.fv32 ? 1 : 0)));
@@ -1605,7 +1638,6 @@ extern "C" int nuc_rhs_noalloc(const nuc_config *cfg, const double *q_dev, doubl
     // from zero (a fill kernel, so that the call can be captured in a graph)
     hipLaunchKernelGGL(k_clear_u64, dim3(1), dim3(256), 0, x.stream, x.lam, (int)NOALLOC_LAM);
     enqueue_stage(&x, 0, 0, 0, false);
-    if (dt_local_dev) hipLaunchKernelGGL(k_copy_dt, dim3(1), dim3(1), 0, x.stream, x.scal, dt_local_dev);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(NUC_EHIP, std::string("launch: ") + hipGetErrorString(e));
     return NUC_OK;
