@@ -623,10 +623,11 @@ int rows_for(int nrows)
 // KB of LDS) leave one wave per SIMD.  Measured, ms a sweep on one -> two
 // waves: 512^3 hccs/AUSM x 17.9 -> 11.2, 512x256^2 CRWENO5 x 3.39 -> 1.98,
 // 512x128^2 WENO5-Z/AUSM x 0.51 -> 0.40, 384x64x384 WENO5-JS z 0.48 -> 0.47.
-// With FP32 stencils (half the LDS and registers) the y and z sweeps stay on
-// one wave, where the larger workgroup's barriers cost more than it gains:
-// 384x64x384 mixed CRWENO5 z 0.47 against 0.53, x 0.51 -> 0.45.
-int sweep_wpl(int n, int dir, bool fp32_stencils) { return n > 256 && (dir == 0 || !fp32_stencils) ? 2 : 1; }
+// FP32 stencils (half the LDS and registers) stay on one wave: y and z lose to
+// the larger workgroup's barriers (384x64x384 mixed CRWENO5 z 0.47 against
+// 0.53), and the rows of a lane decide which products are fused, whose FP32
+// roundings show in the results (x would go 0.51 -> 0.45).
+int sweep_wpl(int n, bool fp32_stencils) { return n > 256 && !fp32_stencils ? 2 : 1; }
 
 // rows per lane of a sweep over a periodic line of n cells: also 3 and 5, so
 // that lines of 65-96 and 129-160 cells (257-320 on two waves) do not leave up
@@ -943,10 +944,10 @@ static void ctx_geometry(nuc_ctx *x, const nuc_config *cfg)
         x->tsv[d] = vis_tilesize(cfg->scheme[d], cfg->vis_scheme[d]);
         x->seg[d] = segment_length(x->n[d], x->nloc[d], x->np[d], cfg->scheme[d]);
         x->nseg[d] = x->n[d] / x->seg[d];
-        // a segment has seg + 1 interfaces: at most 256, or 512 (compact schemes) on two waves
+        // a segment has seg + 1 interfaces: at most 256, or 512 (compact schemes)
         const bool f32s = cfg->precision != NUC_FP64 && cfg->scheme[d] != NUC_HCCS && cfg->scheme[d] != NUC_HCCS77;
-        x->wpl[d] = x->nseg[d] > 1 ? (x->seg[d] > 255 ? 2 : 1) : sweep_wpl(x->n[d], d, f32s);
-        x->cpt[d] = x->nseg[d] > 1 ? 8 : sweep_rows(x->n[d], x->wpl[d]);
+        x->wpl[d] = sweep_wpl(x->nseg[d] > 1 ? x->seg[d] + 1 : x->n[d], f32s);
+        x->cpt[d] = x->nseg[d] > 1 ? (x->seg[d] > 255 && x->wpl[d] == 1 ? 16 : 8) : sweep_rows(x->n[d], x->wpl[d]);
     }
 }
 

@@ -323,19 +323,29 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             T b0, b1, b2, q0, q1, q2, h2;
             w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);
             // the positive inner sweep's is2 reads f_{i+1} twice (src/weno5z.cpp:80):
-            // 13/12 (f2 - f3)^2 in place of its second-difference term
+            // (f2 - f3)^2 in place of its squared second difference
             bool typo = !neg && ml[r] >= z.ts && ml[r] <= z.nloc - z.ts;
-            if (typo) b2 = T(13.0 / 12.0) * sq(d3) + h2 * h2;
+            b2 = (typo ? T(13.0 / 12.0) * sq(d3) : e3) + h2 * h2;
             // alpha_k = c_k (1 + (tau/s_k)^2), s_k = is_k + eps (src/weno5z.cpp:84-92),
             // scaled by s_0^2 s_1^2 s_2^2: no quotient is left but the normalisation
             // (three IEEE quotients are 35 of the plain form's 75 instructions).  The
-            // products hold indicators between eps = 1e-40 and 1e50.
+            // products hold indicators between eps = 1e-40 and 1e50.  FP32 stencils
+            // keep the plain form: with the scaled one the compiler fuses other FP32
+            // products of the rows around it.
             const TW eps = TW(1.0e-40);
             const TW B0 = b0, B1 = b1, B2 = b2;
-            const TW S0 = sq(B0 + eps), S1 = sq(B1 + eps), S2 = sq(B2 + eps), T2 = sq(B2 - B0);
-            const TW a0 = TW(0.1) * ((S0 + T2) * (S1 * S2));
-            const TW a1 = TW(0.6) * ((S1 + T2) * (S0 * S2));
-            const TW a2 = TW(0.3) * ((S2 + T2) * (S0 * S1));
+            TW a0, a1, a2;
+            if constexpr (sizeof(T) == 8) {
+                const TW S0 = sq(B0 + eps), S1 = sq(B1 + eps), S2 = sq(B2 + eps), T2 = sq(B2 - B0);
+                a0 = TW(0.1) * ((S0 + T2) * (S1 * S2));
+                a1 = TW(0.6) * ((S1 + T2) * (S0 * S2));
+                a2 = TW(0.3) * ((S2 + T2) * (S0 * S1));
+            } else {
+                TW tau = fabs(B2 - B0);
+                a0 = TW(0.1) * (TW(1) + sq(tau / (B0 + eps)));
+                a1 = TW(0.6) * (TW(1) + sq(tau / (B1 + eps)));
+                a2 = TW(0.3) * (TW(1) + sq(tau / (B2 + eps)));
+            }
             TS o = TS((a0 * TW(q0) + a1 * TW(q1) + a2 * TW(q2)) * frcp(a0 + a1 + a2));
             pin(o); pin(f3); pin(f4); pin(d3); pin(d4); pin(e2); pin(e3);
             out[r] = o;

@@ -207,7 +207,10 @@ __device__ __forceinline__ void sync_lines(int d)
 // their five parameters to LDS for a fourth wave (WENO5-Z 256^3 x 0.73 -> 0.67,
 // WENO7 160^3 x 0.354 -> 0.337).  Their 8-row form with tails needs 159
 // registers and stays at three waves (230^3 0.72 ms against 0.75 with one
-// parameter in LDS).
+// parameter in LDS).  With FP32 stencils the explicit schemes keep their
+// parameters in registers, which are half as many (and where the parameters are
+// decides which products of the splitting are fused, whose FP32 roundings show
+// in the results).
 template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct SweepForm {
     static constexpr bool COMPACT = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
     static constexpr int NL = 32 * WPL;           // lanes per sign
@@ -218,7 +221,7 @@ template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct
     static constexpr int NP = Skew<R, NL>::pitch(NL * R);
     static constexpr int NV = plain_pitch(NL * R);
     static constexpr bool D64 = sizeof(T) == 8, LF = RIE == RIE_LF;
-    static constexpr bool FREE = R < 5 || R >= 12 || (!COMPACT && D64 && !LF && R == 8 && EPI == EPI_ARG);
+    static constexpr bool FREE = R < 5 || R >= 12 || (!COMPACT && (!D64 || (!LF && R == 8 && EPI == EPI_ARG)));
     static constexpr int WAVES = FREE ? 1 : COMPACT && D64 && (SCH != CRWENO5 || !LF) ? 3 : 4;
     static constexpr int LDS = 163840 * LPB * WPL / (4 * WAVES) - 64;           // bytes of a workgroup
     static constexpr int LINES = LPB * (2 * NP * (int)sizeof(double) + NV * (int)sizeof(T));
@@ -608,16 +611,14 @@ template <int SCH, int RIE, int R, int WPL, bool SEG, typename T, typename S>
 void launch_sweep_rt(const SweepArgs &A, hipStream_t s)
 {
     constexpr int LX = sweep_lpb(WPL, 0, SCH, RIE), LYZ = sweep_lpb(WPL, 1, SCH, RIE);
-    // FP32 stencils sweep x alone on two waves a line (segments: every direction)
-    constexpr bool X_ONLY = WPL == 2 && !SEG && sizeof(T) == 4;
-    if (X_ONLY || LX == LYZ || A.dir == 0) launch_sweep_rtl<SCH, RIE, R, WPL, LX, SEG, T, S>(A, s);
-    else if constexpr (!X_ONLY) launch_sweep_rtl<SCH, RIE, R, WPL, LYZ, SEG, T, S>(A, s);
+    if (LX == LYZ || A.dir == 0) launch_sweep_rtl<SCH, RIE, R, WPL, LX, SEG, T, S>(A, s);
+    else launch_sweep_rtl<SCH, RIE, R, WPL, LYZ, SEG, T, S>(A, s);
 }
 
 template <int SCH, int RIE, int R, int WPL, bool SEG = false>
 void launch_sweep_r(const SweepArgs &A, hipStream_t s)
 {
-    if constexpr (mixed_fp32<SCH>()) {
+    if constexpr (mixed_fp32<SCH>() && WPL == 1) {   // FP32 stencils: one wave a line
         if (A.fp32) {   // NUC_FP32: FP32 state and RHS around the mixed path's arithmetic
             launch_sweep_rt<SCH, RIE, R, WPL, SEG, float, float>(A, s);
             return;
@@ -637,8 +638,11 @@ template <int SCH, int RIE>
 void launch_sweep_sr(int R, const SweepArgs &A, hipStream_t s)
 {
     if (A.nseg > 1) {   // lines longer than 512 cells; whole blocks of 256-511 cells only with the compact schemes
-        if constexpr (compact_scheme(SCH))
+        if constexpr (compact_scheme(SCH)) {
             if (A.wpl == 2) { launch_sweep_r<SCH, RIE, 8, 2, true>(A, s); return; }
+            if constexpr (mixed_fp32<SCH>())
+                if (R == 16) { launch_sweep_r<SCH, RIE, 16, 1, true>(A, s); return; }
+        }
         launch_sweep_r<SCH, RIE, 8, 1, true>(A, s);
         return;
     }
