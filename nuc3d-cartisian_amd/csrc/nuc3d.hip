@@ -286,14 +286,14 @@ __device__ __forceinline__ void gradq_body(const GradArgs &A, int bx, int by, in
     // column's plane k+4 are loaded one plane ahead (ring_q, col_q), so that
     // a plane step does not wait for its own loads: a 512-thread workgroup
     // is alone on its CU at this register count.
-    constexpr int RING_ROWS = 8 * PX;                 // 4 rows above and below the tile
+    constexpr int RING_ROWS = 8 * GTX;                // 4 rows above and below the tile, without the corners
     constexpr int RING = RING_ROWS + GTY * 8;          // + 4 columns left and right
     static_assert(RING <= GTX * GTY, "one ring point per thread");
     const bool has_ring = t < RING;
     int rcx = 0, rcy = 0;
     if (t < RING_ROWS) {
-        rcx = t % PX;
-        rcy = t / PX;
+        rcx = 4 + t % GTX;
+        rcy = t / GTX;
         rcy = rcy < 4 ? rcy : rcy + GTY;
     } else {
         const int u8 = t - RING_ROWS;
@@ -385,7 +385,14 @@ __device__ __forceinline__ void gradq_body(const GradArgs &A, int bx, int by, in
 }
 
 template <typename T, typename S>
-__global__ __launch_bounds__(GTX * GTY) void k_gradq(GradArgs A) { gradq_body<T, S>(A, blockIdx.x, blockIdx.y, blockIdx.z); }
+__global__ __launch_bounds__(GTX * GTY) void k_gradq(GradArgs A)
+{
+    // neighbouring tiles, which share halo cells, on one XCD: 150x132x108 109 ->
+    // 94 us, 128^3 76 -> 72, 97x60x83 38.7 -> 36.2; no change from 160^3 on
+    const unsigned gx = gridDim.x, gy = gridDim.y, p = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const unsigned l = (unsigned)xcd_block(p, gx * gy * gridDim.z), r = l / gx;
+    gradq_body<T, S>(A, l % gx, r % gy, r / gy);
+}
 
 struct ResArgs {
     const double GMEM *part;
