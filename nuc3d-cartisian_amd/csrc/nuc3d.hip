@@ -2914,6 +2914,8 @@ struct nuc_pack {
     bool ns = false, mixed = false, fv32 = false;
     int scheme[3] = {0, 0, 0}, riemann = 0, cpt[3] = {0, 0, 0};
     bool full[3] = {false, false, false};
+    int nj_one[3] = {0, 0, 0};         // sweep jobs of lines of one block, which come first,
+    long sw_one[3] = {0, 0, 0};        // and their workgroups
     bool use_graph = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
@@ -2976,6 +2978,14 @@ extern "C" int nuc_pack_create(nuc_ctx *const *members, int n, int use_graph, nu
     p->fv32 = x0->fv32;
     p->riemann = x0->c.riemann;
     for (int d = 0; d < 3; d++) { p->scheme[d] = x0->c.scheme[d]; p->cpt[d] = x0->cpt[d]; p->full[d] = sweep_full(x0, d); }
+    // the sweeps' jobs: members whose lines are one block first (launch_sweep_pack_rt)
+    std::vector<int> ord[3];
+    for (int d = 0; d < 3; d++) {
+        auto one = [&](int i) { return members[i]->nloc[d] == members[i]->n[d]; };
+        for (int i = 0; i < n; i++) if (one(i)) ord[d].push_back(i);
+        p->nj_one[d] = (int)ord[d].size();
+        for (int i = 0; i < n; i++) if (!one(i)) ord[d].push_back(i);
+    }
     p->use_graph = use_graph != 0;
     auto fail = [&](const char *what, int rc) {
         g_pack_err = what;
@@ -3014,7 +3024,7 @@ extern "C" int nuc_pack_create(nuc_ctx *const *members, int n, int use_graph, nu
         vr[i] = sa[(size_t)2 * n + i].res;
         poff[i + 1] = poff[i] + (int)a0.prim_nb;
         goff[i + 1] = goff[i] + (int)(a0.ggrid.x * a0.ggrid.y * a0.ggrid.z);
-        for (int d = 0; d < 3; d++) soff[d][i + 1] = soff[d][i] + (int)a0.sw_nb[d];
+        for (int d = 0; d < 3; d++) soff[d][i + 1] = soff[d][i] + (int)sa[ord[d][i]].sw_nb[d];
     }
     size_t o_prim = put(vp.data(), sizeof(PrimArgs) * n);
     size_t o_dt = put(vd.data(), sizeof(DtArgs) * n);
@@ -3029,7 +3039,7 @@ extern "C" int nuc_pack_create(nuc_ctx *const *members, int n, int use_graph, nu
         o_grad[st] = put(vg.data(), sizeof(GradArgs) * n);
         for (int d = 0; d < 3; d++) {
             std::vector<SweepArgs> vs(n);
-            for (int i = 0; i < n; i++) vs[i] = sa[(size_t)st * n + i].sw[d];
+            for (int i = 0; i < n; i++) vs[i] = sa[(size_t)st * n + ord[d][i]].sw[d];
             o_sw[st][d] = put(vs.data(), sizeof(SweepArgs) * n);
         }
     }
@@ -3050,7 +3060,7 @@ extern "C" int nuc_pack_create(nuc_ctx *const *members, int n, int use_graph, nu
     }
     p->prim_total = poff[n];
     p->grad_total = goff[n];
-    for (int d = 0; d < 3; d++) p->sw_total[d] = soff[d][n];
+    for (int d = 0; d < 3; d++) { p->sw_total[d] = soff[d][n]; p->sw_one[d] = soff[d][p->nj_one[d]]; }
     *out = p;
     return NUC_OK;
 }
@@ -3075,7 +3085,7 @@ static void pack_enqueue_step(nuc_pack *p)
         }
         for (int i = 0; i < 3; i++) {
             const int d = kSweepOrder[i];
-            PackLaunch L{p->sw[st][d], p->sw_off[d], nj, p->sw_total[d], p->mixed, p->full[d]};
+            PackLaunch L{p->sw[st][d], p->sw_off[d], nj, p->sw_total[d], p->mixed, p->full[d], p->nj_one[d], p->sw_one[d]};
             launch_sweep_pack(p->scheme[d], p->riemann, p->cpt[d], L, p->stream);
         }
         if (st == 2) hipLaunchKernelGGL(k_res_pack, dim3(nj), dim3(256), 0, p->stream, p->res);

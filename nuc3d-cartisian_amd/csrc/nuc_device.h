@@ -37,14 +37,38 @@ __device__ __forceinline__ T w7_sos(T a, T b, T c, T d, bool outer)
     return k0 * e0 * e0 + k1 * e1 * e1 + T(203060.0 / 1063.0) * g2 * g2;
 }
 
-// reciprocal: hardware estimate refined by two Newton steps (|err| <= 1 ulp)
+// reciprocal: hardware estimate r (2^-25 relative) refined by one third-order
+// step, r + r (e + e^2) with e = 1 - x r: e^3 is below 2^-74, and the one
+// rounding left is that of the sum (|err| <= 1 ulp).  Two Newton steps reach the
+// same with one instruction more; the sweeps take 15 reciprocals a variable.
 __device__ __forceinline__ double frcp(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+// Two Newton steps, for the FP64 solve behind FP32 stencils: a last bit of the
+// state that differs moves an FP32 rounding somewhere, and the runs part from
+// there, so these solves keep the reciprocal they have.
+template <bool F32> __device__ __forceinline__ double frcp_for(double x)
+{
+    if constexpr (!F32) {
+        return frcp(x);
+    } else {
+        double r = __builtin_amdgcn_rcp(x);
+        double e = fma(-x, r, 1.0);
+        r = fma(r, e, r);
+        e = fma(-x, r, 1.0);
+        return fma(r, e, r);
+    }
+}
+// a / x from r = 1/x (two Newton steps): the product and one remainder step,
+// which round as the IEEE quotient does, without its scaling (x between 1e-290
+// and 1e290, and finite)
+__device__ __forceinline__ double fquot(double a, double x, double r)
+{
+    const double q = a * r;
+    return fma(fma(-x, q, a), r, q);
 }
 // FP32 (mixed path): the hardware reciprocal, 1 ulp
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -107,6 +131,21 @@ __device__ __forceinline__ TW weno7z(const T *f, TW eps, TW &X)
     weno7_stencil<T>(f, is, q);
     const TW s0 = eps + TW(is[0]), s1 = eps + TW(is[1]), s2 = eps + TW(is[2]), s3 = eps + TW(is[3]);
     const TW tau = fabs(TW(is[0]) - TW(is[3]));
+    if constexpr (sizeof(T) == 4) {
+        // FP32 stencils: the plain form, rounded as its IEEE quotients are (see
+        // frcp_for), with a shared reciprocal for the four of the normalisation.
+        // An indicator beyond FP32's range counts as 1e280 (weight c_k).
+#pragma clang fp contract(off)
+        auto t = [&](TW sk) {
+            const TW x = fmin(sk, TW(1.0e280));
+            return fquot(tau, x, frcp_for<true>(x));
+        };
+        const TW a0 = TW(1.0 / 35.0) * (TW(1) + sq(t(s0))), a1 = TW(12.0 / 35.0) * (TW(1) + sq(t(s1)));
+        const TW a2 = TW(18.0 / 35.0) * (TW(1) + sq(t(s2))), a3 = TW(4.0 / 35.0) * (TW(1) + sq(t(s3)));
+        const TW as = a0 + a1 + a2 + a3, ra = frcp_for<true>(as);
+        X = as - TW(1);
+        return fquot(a0, as, ra) * TW(q[0]) + fquot(a1, as, ra) * TW(q[1]) + fquot(a2, as, ra) * TW(q[2]) + fquot(a3, as, ra) * TW(q[3]);
+    }
     const TW r01 = tau * frcp(s0 * s1), r23 = tau * frcp(s2 * s3);
     const TW x0 = TW(1.0 / 35.0) * sq(r01 * s1), x1 = TW(12.0 / 35.0) * sq(r01 * s0);
     const TW x2 = TW(18.0 / 35.0) * sq(r23 * s3), x3 = TW(4.0 / 35.0) * sq(r23 * s2);
@@ -171,6 +210,7 @@ __device__ __forceinline__ TW weno3js(const T *f)
 
 // hccs interior row, src/hccs.cpp:138-183: Z-type CRWENO weights (eps 1e-40)
 // blended with the 7th-order upwind compact scheme through theta.
+// b0, b1, b2: four times the smoothness indicators; f0..f4 the stencil.
 // T: indicators and stencil values; TW: weights and the row.
 // With S_k = (is_k + eps)^2 the unnormalised weights are c_k (S_k + tau^2)/S_k.
 // Their sum less 1 is X = tau^2 sum_k c_k prod_{j!=k} S_j / (S_0 S_1 S_2),
@@ -178,16 +218,12 @@ __device__ __forceinline__ TW weno3js(const T *f)
 // two reciprocals in place of seven quotients.  The products hold indicators
 // between 1e-40 and 1e50 (fluxes up to about 1e25).
 template <typename T, typename TW>
-__device__ __forceinline__ void hccs_row(T f0, T f1, T f2, T f3, T f4, TW &lo, TW &di, TW &hi, TW &rhs)
+__device__ __forceinline__ void hccs_row(T f0, T f1, T f2, T f3, T f4, T b0, T b1, T b2, TW &lo, TW &di, TW &hi, TW &rhs)
 {
-    const T g0 = T(13.0 / 12.0), g1 = T(0.25);
-    const TW eps = TW(1.0e-40);
-    T is0 = g0 * sq(f0 - T(2) * f1 + f2) + g1 * sq(f0 - T(4) * f1 + T(3) * f2);
-    T is1 = g0 * sq(f1 - T(2) * f2 + f3) + g1 * sq(f1 - f3);
-    T is2 = g0 * sq(f2 - T(2) * f3 + f4) + g1 * sq(T(3) * f2 - T(4) * f3 + f4);
-    T q7 = (-f0 + T(19) * f1 + T(239) * f2 + T(159) * f3 + T(4) * f4) * T(1.0 / 420.0);
-    const TW S0 = sq(TW(is0) + eps), S1 = sq(TW(is1) + eps), S2 = sq(TW(is2) + eps);
-    const TW T2 = sq(TW(is2) - TW(is0));
+    const TW eps = TW(4.0e-40);
+    T q7 = T(-1.0 / 420.0) * f0 + T(19.0 / 420.0) * f1 + T(239.0 / 420.0) * f2 + T(159.0 / 420.0) * f3 + T(4.0 / 420.0) * f4;
+    const TW S0 = sq(TW(b0) + eps), S1 = sq(TW(b1) + eps), S2 = sq(TW(b2) + eps);
+    const TW T2 = sq(TW(b2) - TW(b0));
     const TW P12 = S1 * S2;
     const TW p0 = TW(0.2) * P12, p1 = TW(0.5) * (S0 * S2), p2 = TW(0.3) * (S0 * S1);
     const TW X = (T2 * (p0 + p1 + p2)) * frcp(S0 * P12);

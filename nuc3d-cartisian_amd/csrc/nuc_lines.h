@@ -18,6 +18,8 @@
 #pragma once
 #include "nuc_device.h"
 
+#include <type_traits>
+
 namespace nucdev {
 
 constexpr int HALO = 4;
@@ -29,13 +31,14 @@ struct Zone {
     int off = 0;  // position of interface 0 on the full line (a segment of a long line)
 };
 
-// Unnormalised WENO5 weights n_k ~ c_k / (eps + is_k)^2.  FP64 uses the
-// division-free products c_k * s_i * s_j (one reciprocal per row in total);
-// FP32 uses c_k * rcp(s_k), since the products can leave FP32's range.
+// Unnormalised WENO5 weights n_k ~ c_k / (eps + is_k)^2.  FP64 (b_k = 4 is_k)
+// uses the division-free products c_k * s_i * s_j (one reciprocal per row in
+// total); FP32 (b_k = is_k) uses c_k * rcp(s_k), since the products can leave
+// FP32's range.
 template <typename TW>
 __device__ __forceinline__ void w5_weights(TW b0, TW b1, TW b2, TW c0, TW c1, TW c2, TW &n0, TW &n1, TW &n2)
 {
-    const TW eps = TW(1.0e-6);
+    const TW eps = TW(sizeof(TW) == 8 ? 4.0e-6 : 1.0e-6);
     TW s0 = sq(eps + b0), s1 = sq(eps + b1), s2 = sq(eps + b2);
     if constexpr (sizeof(TW) == 8) {
         n0 = c0 * (s1 * s2); n1 = c1 * (s0 * s2); n2 = c2 * (s0 * s1);
@@ -148,7 +151,7 @@ __device__ __forceinline__ void swap32(double x, double &up, double &dn)
 
 // normalised parallel cyclic reduction over the NL lanes (32 or 64) of one
 // sign: row k: x_k + al*x_{k-1} + ga*x_{k+1} = de  ->  x_k = de on return
-template <int NL, typename T>
+template <int NL, bool F32, typename T>
 __device__ __forceinline__ void pcr(T &al, T &ga, T &de)
 {
 #pragma unroll
@@ -169,7 +172,7 @@ __device__ __forceinline__ void pcr(T &al, T &ga, T &de)
         // exactly (the first and last rows do not couple outward, and each
         // level doubles those ranges), so the values they received from the
         // wrapped or neighbouring lanes, all finite, are multiplied by zero
-        T r = frcp(T(1) - al * gam - ga * alp);
+        T r = frcp_for<F32>(T(1) - al * gam - ga * alp);
         T nal = -r * al * alm;
         T nga = -r * ga * gap;
         T nde = r * (de - al * dem - ga * dep);
@@ -179,15 +182,15 @@ __device__ __forceinline__ void pcr(T &al, T &ga, T &de)
 
 // Forward-eliminated rows of one lane's chunk (rows normalised):
 //   r = 0: Af x_{-1} + x_0 + Cf x_1 = Df ;  r >= 1: Af x_0 + x_r + Cf x_{r+1} = Df
-template <int R, typename T, int NL> struct Chunk {
+template <int R, typename T, int NL, bool F32 = false> struct Chunk {
     T Af[R], Cf[R], Df[R];
     __device__ __forceinline__ void row(int r, T a, T b, T c, T d)
     {
         if (r <= 1) {
-            T rb = frcp(b);
+            T rb = frcp_for<F32>(b);
             Af[r] = a * rb; Cf[r] = c * rb; Df[r] = d * rb;
         } else {
-            T rr = frcp(b - a * Cf[r - 1]);
+            T rr = frcp_for<F32>(b - a * Cf[r - 1]);
             Df[r] = rr * (d - a * Df[r - 1]);
             Af[r] = -rr * a * Af[r - 1];
             Cf[r] = rr * c;
@@ -210,7 +213,7 @@ template <int R, typename T, int NL> struct Chunk {
         if constexpr (R == 2) {
             A0 = Af[0]; C0 = Cf[0]; D0 = Df[0];
         } else {
-            T r0 = frcp(T(1) - Cf[0] * Af[1]);
+            T r0 = frcp_for<F32>(T(1) - Cf[0] * Af[1]);
             A0 = r0 * Af[0];
             C0 = -r0 * Cf[0] * Cf[1];
             D0 = r0 * (Df[0] - Cf[0] * Df[1]);
@@ -218,14 +221,14 @@ template <int R, typename T, int NL> struct Chunk {
         T A1 = Af[R - 1], C1 = Cf[R - 1], D1 = Df[R - 1];
         T A0n = shl1(A0), C0n = shl1(C0), D0n = shl1(D0);
         if (h == NL - 1) { A0n = T(0); C0n = T(0); D0n = T(0); }
-        T rb = frcp(T(1) - A1 * C0 - C1 * A0n);
+        T rb = frcp_for<F32>(T(1) - A1 * C0 - C1 * A0n);
         T al = -rb * A1 * A0;
         T ga = -rb * C1 * C0n;
         T de = rb * (D1 - A1 * D0 - C1 * D0n);
         // the reduced system's first and last rows do not couple outward
         if (h == 0) al = T(0);
         if (h == NL - 1) ga = T(0);
-        pcr<NL>(al, ga, de);
+        pcr<NL, F32>(al, ga, de);
         T X1 = de;
         T X1m = shr1(X1);
         if (h == 0) X1m = T(0);
@@ -240,22 +243,58 @@ template <int R, typename T, int NL> struct Chunk {
 // WENO5 smoothness indicators and candidate values of a 5-point upwind stencil
 // f0..f4 (src/weno5js.cpp, src/crweno5.cpp:87-129), computed from the
 // stencil's differences d_j = f_j - f_{j-1} (j = 1..4) and second-difference
-// terms e_k = 13/12 (d_{k+1} - d_k)^2 (k = 1..3), which a lane's consecutive
+// terms e_k = 13/3 (d_{k+1} - d_k)^2 (k = 1..3), which a lane's consecutive
 // rows share: f0-4f1+3f2 = 3d2-d1, f1-f3 = -(d2+d3), 3f2-4f3+f4 = d4-3d3,
-// q0 = f2+(5d2-2d1)/6, q1 = f2+(d2+2d3)/6, q2 = f3-(2d3+d4)/6.  The linear
-// parts are halved (h_k), so that b_k = e_k + h_k^2 with the 1/4 folded in.
+// q0 = f2+(5d2-2d1)/6, q1 = f2+(d2+2d3)/6, q2 = f3-(2d3+d4)/6.  In FP64 the
+// indicators come as b_k = e_k + (linear part)^2, four times is_k: the factor 1/4
+// of the linear parts would be three more multiplications, and the weights only
+// need the indicators' ratios (their eps is taken times four as well).  In FP32
+// the linear parts are halved (b_k = is_k): the roundings of an FP32 stencil are
+// seen in the results, so they stay what they were.
+template <typename T> constexpr bool W5_FOUR = sizeof(T) == 8;   // b_k = 4 is_k
+template <typename T> constexpr T w5_g() { return T(W5_FOUR<T> ? 13.0 / 3.0 : 13.0 / 12.0); }
+// h2: the linear part of b2
 template <typename T>
 __device__ __forceinline__ void w5_diff(T f2, T f3, T d1, T d2, T d3, T d4, T e1, T e2, T e3, T &b0, T &b1, T &b2,
                                         T &q0, T &q1, T &q2, T &h2)
 {
-    const T h0 = T(1.5) * d2 - T(0.5) * d1, h1 = T(0.5) * (d2 + d3);
-    h2 = T(0.5) * d4 - T(1.5) * d3;
-    b0 = e1 + h0 * h0;
-    b1 = e2 + h1 * h1;
-    b2 = e3 + h2 * h2;
+    if constexpr (W5_FOUR<T>) {
+        const T h0 = T(3) * d2 - d1, h1 = d2 + d3;
+        h2 = d4 - T(3) * d3;
+        b0 = e1 + h0 * h0;
+        b1 = e2 + h1 * h1;
+        b2 = e3 + h2 * h2;
+    } else {
+        const T h0 = T(1.5) * d2 - T(0.5) * d1, h1 = T(0.5) * (d2 + d3);
+        h2 = T(0.5) * d4 - T(1.5) * d3;
+        b0 = e1 + h0 * h0;
+        b1 = e2 + h1 * h1;
+        b2 = e3 + h2 * h2;
+    }
     q0 = f2 + (T(5.0 / 6.0) * d2 - T(1.0 / 3.0) * d1);
     q1 = f2 + (T(1.0 / 6.0) * d2 + T(1.0 / 3.0) * d3);
     q2 = f3 - (T(1.0 / 3.0) * d3 + T(1.0 / 6.0) * d4);
+}
+
+// The explicit rows of a compact line of one block (2 ts + 1 around interfaces
+// 0 and nloc, ts the scheme's own tilesize), numbered k = 0 .. 2 (2 ts + 1) - 1:
+// the interface m of row k; its place in row order is m of f^+, NL R - 1 - m of f^-.
+template <int SCH> constexpr int edge_ts() { return SCH == HCCS ? 4 : 3; }
+// Their values are kept in the pad slots of the line's buffer (one after every R
+// positions, Skew<R>), which nothing else uses: row k in slot edge_slot(k).
+template <int R, int NL> __host__ __device__ constexpr int edge_slot(int k)
+{
+    static_assert(17 * (R + 1) + R < Skew<R, NL>::span(NL * R), "a pad slot for every explicit row");
+    return k * (R + 1) + R;
+}
+template <int SCH> __device__ __forceinline__ int edge_row(const Zone &z, int k)
+{
+    constexpr int ts = edge_ts<SCH>(), ne = 2 * ts + 1;
+    return k < ne ? k - ts : z.nloc + k - ne - ts;
+}
+template <int SCH> __device__ __forceinline__ bool edge_mine(const Zone &z, int k, int m)
+{
+    return k < 2 * (2 * edge_ts<SCH>() + 1) && m >= 0 && m <= z.nloc;
 }
 
 // Reconstruct one sign of a line.  Lw points at the lane's window in the
@@ -268,15 +307,22 @@ __device__ __forceinline__ void w5_diff(T f2, T f3, T d1, T d2, T d3, T d4, T e1
 // tridiagonal solve and of the result (FP64 in both precision paths).
 // NL: lanes per sign, h in [0, NL).
 // full: every row of every lane is an interface of the line (n = NL R).
-template <int SCH, int R, typename T, typename TW, typename TS, int NL = 32>
+// EDGE_AHEAD (the line is one block): the explicit rows of CRWENO5 and hccs are
+// evaluated ahead.  They are then in slot edge_slot(k) of the wave's and sign's
+// line buffer Lx, and out[] of those rows is meaningless.
+// tails: rows past the line's last interface read defined (finite) cells.
+enum { EDGE_IN_LOOP = 0, EDGE_AHEAD = 1 };
+template <int SCH, int R, typename T, typename TW, typename TS, int NL = 32, int EDGE = EDGE_IN_LOOP>
 __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const Zone &z, int h, bool neg,
-                                          TS out[R], bool full = false)
+                                          TS out[R], bool full = false, TS *Lx = nullptr, bool tails = false)
 {
     constexpr int RAD = Radius<SCH>::value;
     constexpr int W = R + 2 * RAD + Extra<SCH>::value;
     T win[W];
+    if constexpr (EDGE == EDGE_IN_LOOP) {
 #pragma unroll
-    for (int t = 0; t < W; t++) win[t] = Lw[Skew<R>::at(t - RAD - 1)];
+        for (int t = 0; t < W; t++) win[t] = Lw[Skew<R>::at(t - RAD - 1)];
+    }
     // rank-local position of each row, without integer division in the loop
     int ml[R];
     {
@@ -294,12 +340,12 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // rows in order through a rolling window of differences (see CRWENO5)
         T f2 = win[2], f3 = win[3];
         T d1 = win[1] - win[0], d2 = f2 - win[1], d3 = f3 - f2;
-        T e1 = T(13.0 / 12.0) * sq(d2 - d1), e2 = T(13.0 / 12.0) * sq(d3 - d2);
+        T e1 = w5_g<T>() * sq(d2 - d1), e2 = w5_g<T>() * sq(d3 - d2);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             T f4 = win[r + 4];
             T d4 = f4 - f3;
-            T e3 = T(13.0 / 12.0) * sq(d4 - d3);
+            T e3 = w5_g<T>() * sq(d4 - d3);
             T b0, b1, b2, q0, q1, q2, h2;
             w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);
             // alpha_k = c_k / s_k, normalised with a single reciprocal
@@ -314,25 +360,24 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // rows in order through a rolling window of differences (see CRWENO5)
         T f2 = win[2], f3 = win[3];
         T d1 = win[1] - win[0], d2 = f2 - win[1], d3 = f3 - f2;
-        T e1 = T(13.0 / 12.0) * sq(d2 - d1), e2 = T(13.0 / 12.0) * sq(d3 - d2);
+        T e1 = w5_g<T>() * sq(d2 - d1), e2 = w5_g<T>() * sq(d3 - d2);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             T f4 = win[r + 4];
             T d4 = f4 - f3;
-            T e3 = T(13.0 / 12.0) * sq(d4 - d3);
+            T e3 = w5_g<T>() * sq(d4 - d3);
             T b0, b1, b2, q0, q1, q2, h2;
             w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);
             // the positive inner sweep's is2 reads f_{i+1} twice (src/weno5z.cpp:80):
             // (f2 - f3)^2 in place of its squared second difference
             bool typo = !neg && ml[r] >= z.ts && ml[r] <= z.nloc - z.ts;
-            b2 = (typo ? T(13.0 / 12.0) * sq(d3) : e3) + h2 * h2;
+            b2 = (typo ? w5_g<T>() * sq(d3) : e3) + h2 * h2;
             // alpha_k = c_k (1 + (tau/s_k)^2), s_k = is_k + eps (src/weno5z.cpp:84-92),
             // scaled by s_0^2 s_1^2 s_2^2: no quotient is left but the normalisation
             // (three IEEE quotients are 35 of the plain form's 75 instructions).  The
             // products hold indicators between eps = 1e-40 and 1e50.  FP32 stencils
-            // keep the plain form: with the scaled one the compiler fuses other FP32
-            // products of the rows around it.
-            const TW eps = TW(1.0e-40);
+            // keep the plain form and its roundings (weno7z).
+            const TW eps = TW(W5_FOUR<T> ? 4.0e-40 : 1.0e-40);
             const TW B0 = b0, B1 = b1, B2 = b2;
             TW a0, a1, a2;
             if constexpr (sizeof(T) == 8) {
@@ -342,11 +387,15 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
                 a2 = TW(0.3) * ((S2 + T2) * (S0 * S1));
             } else {
                 TW tau = fabs(B2 - B0);
-                a0 = TW(0.1) * (TW(1) + sq(tau / (B0 + eps)));
-                a1 = TW(0.6) * (TW(1) + sq(tau / (B1 + eps)));
-                a2 = TW(0.3) * (TW(1) + sq(tau / (B2 + eps)));
+                auto t = [&](TW s) {
+                    const TW x = fmin(s, TW(1.0e280));   // an indicator beyond FP32's range
+                    return fquot(tau, x, frcp_for<true>(x));
+                };
+                a0 = TW(0.1) * (TW(1) + sq(t(B0 + eps)));
+                a1 = TW(0.6) * (TW(1) + sq(t(B1 + eps)));
+                a2 = TW(0.3) * (TW(1) + sq(t(B2 + eps)));
             }
-            TS o = TS((a0 * TW(q0) + a1 * TW(q1) + a2 * TW(q2)) * frcp(a0 + a1 + a2));
+            TS o = TS((a0 * TW(q0) + a1 * TW(q1) + a2 * TW(q2)) * frcp_for<sizeof(T) == 4>(a0 + a1 + a2));
             pin(o); pin(f3); pin(f4); pin(d3); pin(d4); pin(e2); pin(e3);
             out[r] = o;
             f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;
@@ -392,8 +441,10 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
 #pragma unroll
             for (int j = 0; j < 7; j++) fw[j] = fw[j + 1];
         }
-    } else if constexpr (SCH == CRWENO5) {
-        Chunk<R, TS, NL> ch;
+    } else if constexpr (SCH == CRWENO5 && sizeof(T) == 4) {
+        // FP32 stencils: the explicit rows in place (see below; their FP32
+        // arithmetic costs half, and no form of them ahead was faster)
+        Chunk<R, TS, NL, true> ch;
         // Rows in order: a rolling window (f1..f4, the differences d1..d4 and
         // the second-difference terms e1..e3 of the current row), where the
         // values the next row reuses and the row's own coefficients pass
@@ -403,12 +454,12 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // 2 waves per SIMD, against 164 and 3 waves in order).
         T f1 = win[1], f2 = win[2], f3 = win[3];
         T d1 = f1 - win[0], d2 = f2 - f1, d3 = f3 - f2;
-        T e1 = T(13.0 / 12.0) * sq(d2 - d1), e2 = T(13.0 / 12.0) * sq(d3 - d2);
+        T e1 = w5_g<T>() * sq(d2 - d1), e2 = w5_g<T>() * sq(d3 - d2);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             T f4 = win[r + 4];
             T d4 = f4 - f3;
-            T e3 = T(13.0 / 12.0) * sq(d4 - d3);
+            T e3 = w5_g<T>() * sq(d4 - d3);
             T b0, b1, b2, q0, q1, q2, h2;
             w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);
             TW P0, P1, P2;   // weights with unit ideal weights
@@ -447,6 +498,137 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         ch.solve(h);
 #pragma unroll
         for (int r = 0; r < R; r++) out[r] = ch.Df[r];
+    } else if constexpr (SCH == CRWENO5 || SCH == HCCS) {
+        // The explicit rows (2 ts + 1 around every block edge) lie in a few
+        // lanes only, but evaluated in the row loop every row of every wave pays
+        // for them: 27 of CRWENO5's 97 instructions a row (the candidate values,
+        // the explicit row, the choice between the two), 150 of hccs's.  On a
+        // line of one block lane h evaluates the h-th of them ahead, and the
+        // rows next to them take their values to the right-hand side.  The rows
+        // the loop still forms at their places are ordinary compact rows that no
+        // other row reads.
+        // Measured with the shorter indicators and reciprocals of the same rows, us
+        // x/y/z: CRWENO5/LF 192^3 367/412/414 -> 361/400/385, 256^3 818/903/885 ->
+        // 825/851/836 (the x sweep, which applies the update, spills 12 registers
+        // either way), with AUSM 914/968/950 -> 862/914/890; hccs/LF 256^3
+        // 1220/1212/1184 -> 1133/1130/1118.
+        constexpr int RAD5 = 2;   // the 5-point stencil's window is win[O..]
+        constexpr int O = RAD - RAD5;
+        Chunk<R, TS, NL> ch;
+        constexpr bool AHEAD = EDGE == EDGE_AHEAD;
+        if constexpr (AHEAD) {
+            const T *const Lb = Lw - h * (R + 1);
+            const int m = edge_row<SCH>(z, h);
+            const int y = !edge_mine<SCH>(z, h, m) ? 0 : (neg ? NL * R - 1 - m : m);
+            T fe[2 * RAD + 1];
+#pragma unroll
+            for (int j = 0; j < 2 * RAD + 1; j++) fe[j] = Lb[Skew<R>::at(y - RAD - 1 + j)];
+            TS x;
+            if constexpr (SCH == HCCS) {
+                x = TS(weno7z<T, TW>(fe, TW(1.0e-40)));
+            } else {
+                const T c1 = fe[1] - fe[0], c2 = fe[2] - fe[1], c3 = fe[3] - fe[2], c4 = fe[4] - fe[3];
+                const T k1 = w5_g<T>() * sq(c2 - c1), k2 = w5_g<T>() * sq(c3 - c2), k3 = w5_g<T>() * sq(c4 - c3);
+                T b0, b1, b2, q0, q1, q2, h2;
+                w5_diff<T>(fe[2], fe[3], c1, c2, c3, c4, k1, k2, k3, b0, b1, b2, q0, q1, q2, h2);
+                TW P0, P1, P2;
+                w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);
+                const TW n0 = TW(0.1) * P0, n1 = TW(0.6) * P1, n2 = TW(0.3) * P2;
+                x = TS(n0 * TW(q0) + n1 * TW(q1) + n2 * TW(q2)) * frcp(TS(n0 + n1 + n2));
+            }
+            if (h < 2 * (2 * edge_ts<SCH>() + 1)) Lx[edge_slot<R, NL>(h)] = x;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // the window is read after the explicit rows, whose registers it takes
+            asm volatile("; explicit rows ahead" ::: "memory");
+#pragma unroll
+            for (int t = 0; t < W; t++) win[t] = Lw[Skew<R>::at(t - RAD - 1)];
+        }
+        // rows in order, as above
+        T f1 = win[O + 1], f2 = win[O + 2], f3 = win[O + 3];
+        T d1 = f1 - win[O], d2 = f2 - f1, d3 = f3 - f2;
+        T e1 = w5_g<T>() * sq(d2 - d1), e2 = w5_g<T>() * sq(d3 - d2);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            T f4 = win[O + r + 4];
+            T d4 = f4 - f3;
+            T e3 = w5_g<T>() * sq(d4 - d3);
+            T b0, b1, b2, q0, q1, q2, h2;
+            w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);
+            // Every row is scaled by a factor of its own, which leaves the
+            // tridiagonal solution unchanged: the compact row
+            // (src/crweno5.cpp:133-162) by 3 times the weight denominator, the
+            // explicit WENO5-JS closure (src/crweno5.cpp:87-129) as the row
+            // (sum n_k) x = sum n_k q_k with the unnormalised JS weights n_k.
+            TW lo, di, hi, rhs;
+            TW be = TW(0), de = TW(0);   // the explicit row, formed in place
+            TW P0, P1, P2;   // weights with unit ideal weights
+            if constexpr (SCH == HCCS) {
+                hccs_row<T, TW>(f1 - d1, f1, f2, f3, f4, b0, b1, b2, lo, di, hi, rhs);
+            } else {
+                w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);
+                if constexpr (!AHEAD) {
+                    const TW n0 = TW(0.1) * P0, n1 = TW(0.6) * P1, n2 = TW(0.3) * P2;
+                    be = n0 + n1 + n2;
+                    de = n0 * TW(q0) + n1 * TW(q1) + n2 * TW(q2);
+                }
+                TW m0 = TW(0.2) * P0, m1 = TW(0.5) * P1, m2 = TW(0.3) * P2;
+                lo = TW(2) * m0 + m1;
+                di = m0 + TW(2) * (m1 + m2);
+                hi = m2;
+                rhs = (m0 * TW(f1) + (TW(5) * (m0 + m1) + m2) * TW(f2) + (m1 + TW(5) * m2) * TW(f3)) * TW(0.5);
+            }
+            TS a = TS(lo), b = TS(di), c = TS(hi), d = TS(rhs);
+            const bool valid = full || tails || m0r + mstep * r < z.nrows;
+            if constexpr (AHEAD) {
+                // the block's first and last compact rows, in row order: of a
+                // full line (n = NL R) they can only be these r
+                constexpr int ts = edge_ts<SCH>();
+                if (!full || r == (ts + 1) % R || r == ts % R || r == (NL * R - ts - 1) % R || r == (NL * R - ts - 2) % R) {
+                    const bool first = ml[r] == (neg ? z.nloc - ts - 1 : ts + 1);
+                    const bool last = ml[r] == (neg ? ts + 1 : z.nloc - ts - 1);
+                    // the explicit rows before and after, in row order
+                    const TS xlo = Lx[edge_slot<R, NL>(2 * ts)], xhi = Lx[edge_slot<R, NL>(2 * ts + 1)];
+                    const TS xp = neg ? xhi : xlo, xn = neg ? xlo : xhi;
+                    d -= (first ? a : TS(0)) * xp + (last ? c : TS(0)) * xn;
+                    if (first) a = TS(0);
+                    if (last) c = TS(0);
+                }
+                if (!valid) { a = TS(0); b = TS(1); c = TS(0); d = TS(0); }
+            } else {
+                const bool expl = ml[r] <= z.ts || ml[r] >= z.nloc - z.ts;
+                if constexpr (SCH == HCCS) {
+                    // through the asm as well, so that the rows' WENO7 values
+                    // are formed one after the other
+                    T fw[7];
+#pragma unroll
+                    for (int j = 0; j < 7; j++) { fw[j] = win[r + j]; pin(fw[j]); }
+                    TS x = TS(0);
+                    if (expl) x = TS(weno7z<T, TW>(fw, TW(1.0e-40)));
+                    pin(x);
+                    if (expl) { a = TS(0); b = TS(1); c = TS(0); d = x; }
+                    if (!valid) { a = TS(0); b = TS(1); c = TS(0); d = TS(0); }
+                } else {
+                    a = (valid && !expl) ? TS(lo) : TS(0);
+                    b = valid ? TS(expl ? be : di) : TS(1);
+                    c = (valid && !expl) ? TS(hi) : TS(0);
+                    d = valid ? TS(expl ? de : rhs) : TS(0);
+                }
+            }
+            // the previous row's elimination step is done before this row's
+            // coefficients are released, so that rows do not queue up for it
+            if (r > 0) {
+                pin(ch.Af[r - 1]); pin(ch.Cf[r - 1]); pin(ch.Df[r - 1]);
+            }
+            asm volatile("" : "+v"(f2), "+v"(f3), "+v"(f4), "+v"(d3), "+v"(d4), "+v"(e2), "+v"(e3),
+                              "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+            ch.row(r, a, b, c, d);
+            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;
+        }
+        ch.solve(h);
+#pragma unroll
+        for (int r = 0; r < R; r++) out[r] = ch.Df[r];
     } else if constexpr (SCH == HCCS77) {
         // compact rows on ts+1..nloc-ts-1, WENO7-Z rows at ts and nloc-ts and
         // on the edges (src/hccs77.cpp:86-163, :349-455)
@@ -463,60 +645,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             bool expl = ml[r] <= z.ts || ml[r] >= z.nloc - z.ts;
             TW a, b, c, d;
             hccs77_row<T, TW>(f, expl, a, b, c, d);
-            if (!valid) { a = TW(0); b = TW(1); c = TW(0); d = TW(0); }
-            TS as = TS(a), bs = TS(b), cs = TS(c), ds = TS(d);
-            if (r > 0) {
-                pin(ch.Af[r - 1]); pin(ch.Cf[r - 1]); pin(ch.Df[r - 1]);
-            }
-            pin(as); pin(bs); pin(cs); pin(ds);
-#pragma unroll
-            for (int j = 1; j < 7; j++) pin(fw[j]);
-            ch.row(r, as, bs, cs, ds);
-#pragma unroll
-            for (int j = 0; j < 6; j++) fw[j] = fw[j + 1];
-        }
-        ch.solve(h);
-#pragma unroll
-        for (int r = 0; r < R; r++) out[r] = ch.Df[r];
-    } else {  // HCCS
-        Chunk<R, TS, NL> ch;
-        // The explicit WENO7-Z rows (2 ts + 1 around every rank-block edge) lie
-        // in a few lanes only.  Evaluated in the row loop, all R rows of every
-        // wave pay for them (about 150 instructions each).  Lines of up to two
-        // blocks have at most 27 of them: lane h evaluates the h-th, and leaves
-        // its value at the interface's place in the line buffer, whose windows
-        // are in registers by then.
-        T *const Lb = const_cast<T *>(Lw) - h * (R + 1);
-        const int ne = 2 * z.ts + 1, nexp = (z.nrows / z.nloc + 1) * ne;
-        const bool ahead = nexp <= NL;
-        if (ahead) {
-            const int e = h / ne, m = e * z.nloc + (h - e * ne) - z.ts;   // interface of the h-th row
-            const bool mine = h < nexp && m >= 0 && m < z.nrows;
-            const int y = !mine ? 0 : (neg ? NL * R - 1 - m : m);         // its position in the lane order
-            T fe[7];
-#pragma unroll
-            for (int j = 0; j < 7; j++) fe[j] = Lb[Skew<R>::at(y - 4 + j)];
-            TW x = weno7z<T, TW>(fe, TW(1.0e-40));
-            pin(x);
-#pragma unroll
-            for (int t = 0; t < W; t++) pin(win[t]);
-            if (mine) Lb[Skew<R>::at(y)] = T(x);
-            __builtin_amdgcn_wave_barrier();
-        }
-        T fw[7];   // 7-point window for the closures, 5-point from fw+1
-#pragma unroll
-        for (int j = 0; j < 6; j++) fw[j] = win[j];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            fw[6] = win[r + 6];
-            const T *f = fw;
-            int m = m0r + mstep * r;
-            bool valid = full || m < z.nrows;
-            bool expl = ml[r] <= z.ts || ml[r] >= z.nloc - z.ts;
-            TW a, b, c, d, x = TW(Lw[Skew<R>::at(r)]);
-            if (!ahead && valid && expl) x = weno7z<T, TW>(f, TW(1.0e-40));
-            hccs_row<T, TW>(f[1], f[2], f[3], f[4], f[5], a, b, c, d);
-            if (expl || !valid) { a = TW(0); b = TW(1); c = TW(0); d = valid ? x : TW(0); }
+            if (!valid && !tails) { a = TW(0); b = TW(1); c = TW(0); d = TW(0); }
             TS as = TS(a), bs = TS(b), cs = TS(c), ds = TS(d);
             if (r > 0) {
                 pin(ch.Af[r - 1]); pin(ch.Cf[r - 1]); pin(ch.Df[r - 1]);

@@ -211,7 +211,7 @@ __device__ __forceinline__ void sync_lines(int d)
 // parameters in registers, which are half as many (and where the parameters are
 // decides which products of the splitting are fused, whose FP32 roundings show
 // in the results).
-template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct SweepForm {
+template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL, int EDGE> struct SweepForm {
     static constexpr bool COMPACT = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
     static constexpr int NL = 32 * WPL;           // lanes per sign
     static constexpr int GS = 64 * WPL;           // threads per line in the load mapping
@@ -223,7 +223,8 @@ template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct
     static constexpr bool D64 = sizeof(T) == 8, LF = RIE == RIE_LF;
     static constexpr bool FREE = R < 5 || R >= 12 || (!COMPACT && (!D64 || (!LF && R == 8 && EPI == EPI_ARG)));
     static constexpr int WAVES = FREE ? 1 : COMPACT && D64 && (SCH != CRWENO5 || !LF) ? 3 : 4;
-    static constexpr int LDS = 163840 * LPB * WPL / (4 * WAVES) - 64;           // bytes of a workgroup
+    // bytes of a workgroup: LDS is given out in 128 parts of 1280 bytes
+    static constexpr int LDS = 128 * LPB * WPL / (4 * WAVES) * 1280 - 64;
     static constexpr int LINES = LPB * (2 * NP * (int)sizeof(double) + NV * (int)sizeof(T));
     static constexpr int SPB = CPL * GS * LPB * (int)sizeof(T);               // one split parameter of every cell
     static constexpr int FIT = (LDS - LINES) / SPB < 0 ? 0 : (LDS - LINES) / SPB;
@@ -248,11 +249,12 @@ template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL> struct
 // whole line; the 2*HALO cells around the segment are read from the
 // neighbouring segments (periodic over the full line) and the segment's n+1
 // interfaces are all computed, so that no periodic image is needed.
-template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1>
+template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1,
+          int EDGE = EDGE_IN_LOOP>
 __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
 {
     const bool epi = EPI == EPI_ARG ? A.epilogue != 0 : EPI == EPI_YES;
-    using F = SweepForm<SCH, RIE, R, LPB, T, EPI, WPL>;
+    using F = SweepForm<SCH, RIE, R, LPB, T, EPI, WPL, EDGE>;
     constexpr int NL = F::NL, GS = F::GS, CPL = F::CPL, NSP = F::NSP, NP = F::NP, NV = F::NV, NLD = F::NLD;
     using Sk = Skew<R, NL>;
     constexpr int RAD = Radius<SCH>::value;
@@ -377,6 +379,17 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     const int mstep = neg ? -1 : 1;
     double res = 0.0;
     const double dt = epi ? *A.dtp : 0.0;
+    // The compact schemes' rows past the line's last interface: with FP64 line
+    // buffers the cells they read are set to zero here and never written again
+    // (the interface values stay below them), so that these rows are finite and
+    // need no replacement; the line's last row does not couple to them.
+    constexpr bool TAILS = F::COMPACT && !FULL && sizeof(T) == 8;
+    if constexpr (TAILS) {
+        for (int c = n + HALO + g; c <= NL * R + 2; c += GS) {
+            Pl[Sk::at(c)] = T(0);
+            Ml[Sk::mir(c)] = T(0);
+        }
+    }
 
     // global loads of variable v (state and viscous flux) are issued one
     // variable ahead, so that they are in flight during the previous
@@ -459,7 +472,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         // with eps down to 1e-40 and stay FP64
         constexpr bool zw = SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78;
         using TW = typename std::conditional<zw, double, T>::type;
-        if (wv) line_half<SCH, R, T, TW, double, NL>(Lw, m0r, mstep, z, h, neg, out, FULL);
+        if (wv) line_half<SCH, R, T, TW, double, NL, EDGE>(Lw, m0r, mstep, z, h, neg, out, FULL, neg ? Mw : Pw, TAILS);
         // the interface values overwrite the wave's own line only: the
         // reconstruction of the other waves is not waited for
         sync_wave();
@@ -482,6 +495,15 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
             if constexpr (!SEG) {
                 if (!neg && h == 0) Pw[Sk::at(n)] = out[0];
                 if (neg && h == NL - 1) Mw[Sk::mir(n)] = out[R - 1];
+            }
+            // the explicit rows evaluated ahead (interface n of a periodic line
+            // among them): row y of f^- goes to the slot of y - 1, as its rows do.
+            // They replace what the loop's rows left there.
+            if constexpr (EDGE == EDGE_AHEAD) {
+                sync_wave();
+                const int m = edge_row<SCH>(z, h);
+                double *const Lx = neg ? Mw : Pw;
+                if (edge_mine<SCH>(z, h, m)) Lx[Sk::at(neg ? NL * R - 2 - m : m)] = Lx[edge_slot<R, NL>(h)];
             }
         }
         if constexpr (!F::PREF) fetch(v + 1, qnx, xnx);
@@ -553,10 +575,11 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     }
 }
 
-template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1>
-__global__ __launch_bounds__(64 * LPB * WPL, (SweepForm<SCH, RIE, R, LPB, T, EPI, WPL>::WAVES)) void k_sweep(SweepArgs A)
+template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EPI, typename S = double, bool SEG = false, int WPL = 1,
+          int EDGE = EDGE_IN_LOOP>
+__global__ __launch_bounds__(64 * LPB * WPL, (SweepForm<SCH, RIE, R, LPB, T, EPI, WPL, EDGE>::WAVES)) void k_sweep(SweepArgs A)
 {
-    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI, S, SEG, WPL>(A, xcd_block(blockIdx.x, gridDim.x));
+    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI, S, SEG, WPL, EDGE>(A, xcd_block(blockIdx.x, gridDim.x));
 }
 
 constexpr int SWEEP_LPB = 4;
@@ -588,23 +611,41 @@ constexpr int sweep_lpb(int wpl, int dir, int sch, int rie) { return wpl == 1 ? 
 // the kernel forms for one state type S and stencil type T: FULL kernels
 // (every lane's rows on the line, even R) with and without the RK3 update,
 // else the one that takes it as an argument
-template <int SCH, int RIE, int R, int WPL, int LPB, bool SEG, typename T, typename S>
-void launch_sweep_rtl(const SweepArgs &A, hipStream_t s)
+template <int SCH, int RIE, int R, int WPL, int LPB, bool SEG, typename T, typename S, int EDGE>
+void launch_sweep_rtle(const SweepArgs &A, hipStream_t s)
 {
     const dim3 grid((unsigned)((A.nlines * A.nseg + LPB - 1) / LPB)), block(64 * LPB * WPL);
     // odd R: the load mapping's cells overrun the line, so no FULL form
     if constexpr (!SEG && R % 2 == 0) {
         const bool full = A.n == 32 * WPL * R && A.nlines % LPB == 0;
         if (full && A.epilogue) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_YES, S, false, WPL>), grid, block, 0, s, A);
+            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_YES, S, false, WPL, EDGE>), grid, block, 0, s, A);
             return;
         }
         if (full) {
-            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_NO, S, false, WPL>), grid, block, 0, s, A);
+            hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, true, EPI_NO, S, false, WPL, EDGE>), grid, block, 0, s, A);
             return;
         }
     }
-    hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, false, EPI_ARG, S, SEG, WPL>), grid, block, 0, s, A);
+    hipLaunchKernelGGL((k_sweep<SCH, RIE, R, LPB, T, false, EPI_ARG, S, SEG, WPL, EDGE>), grid, block, 0, s, A);
+}
+
+// CRWENO5 and hccs lines of one block evaluate their explicit rows ahead
+// (line_half); a line of several blocks (from four on they are more than a wave
+// has lanes) forms them in the row loop.  With two rows a lane the loop has two
+// rows to save on and pays one ahead; FP32 stencils save half as much and gained
+// nothing (256^3 mixed 644/745/760 us ahead, 648/744/759 in place).
+template <int SCH, int R, typename T> constexpr bool edge_scheme() { return (SCH == CRWENO5 || SCH == HCCS) && R > 2 && sizeof(T) == 8; }
+template <int SCH, int RIE, int R, int WPL, int LPB, bool SEG, typename T, typename S>
+void launch_sweep_rtl(const SweepArgs &A, hipStream_t s)
+{
+    if constexpr (edge_scheme<SCH, R, T>() && !SEG) {
+        if (A.nloc == A.nfull) {
+            launch_sweep_rtle<SCH, RIE, R, WPL, LPB, SEG, T, S, EDGE_AHEAD>(A, s);
+            return;
+        }
+    }
+    launch_sweep_rtle<SCH, RIE, R, WPL, LPB, SEG, T, S, EDGE_IN_LOOP>(A, s);
 }
 
 template <int SCH, int RIE, int R, int WPL, bool SEG, typename T, typename S>
@@ -687,12 +728,12 @@ __device__ __forceinline__ int pack_job(const int *off, int nj, long b)
     return j;
 }
 
-template <int SCH, int RIE, int R, int LPB, typename T, bool FULL>
+template <int SCH, int RIE, int R, int LPB, typename T, bool FULL, int EDGE>
 __global__ __launch_bounds__(64 * LPB) void k_sweep_pack(const SweepArgs *__restrict__ tab, const int *__restrict__ off, int nj)
 {
-    const long b = xcd_block(blockIdx.x, gridDim.x);
+    const long b = off[0] + xcd_block(blockIdx.x, gridDim.x);
     const int j = pack_job(off, nj, b);
-    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI_ARG>(tab[j], b - off[j]);
+    sweep_body<SCH, RIE, R, LPB, T, FULL, EPI_ARG, double, false, 1, EDGE>(tab[j], b - off[j]);
 }
 
 struct PackLaunch {
@@ -701,19 +742,36 @@ struct PackLaunch {
     int nj;
     long nblocks;
     bool mixed, full;
+    int nj_one;        // the jobs whose lines are one block each come first,
+    long nblocks_one;  // and these are their workgroups
 };
 
-template <int SCH, int RIE, int R, typename T>
-void launch_sweep_pack_rt(const PackLaunch &P, hipStream_t s)
+template <int SCH, int RIE, int R, typename T, int EDGE>
+void launch_sweep_pack_rte(const PackLaunch &P, hipStream_t s)
 {
     const dim3 grid((unsigned)P.nblocks), block(64 * SWEEP_LPB);
     if constexpr (R % 2 == 0) {
         if (P.full) {
-            hipLaunchKernelGGL((k_sweep_pack<SCH, RIE, R, SWEEP_LPB, T, true>), grid, block, 0, s, P.tab, P.off, P.nj);
+            hipLaunchKernelGGL((k_sweep_pack<SCH, RIE, R, SWEEP_LPB, T, true, EDGE>), grid, block, 0, s, P.tab, P.off, P.nj);
             return;
         }
     }
-    hipLaunchKernelGGL((k_sweep_pack<SCH, RIE, R, SWEEP_LPB, T, false>), grid, block, 0, s, P.tab, P.off, P.nj);
+    hipLaunchKernelGGL((k_sweep_pack<SCH, RIE, R, SWEEP_LPB, T, false, EDGE>), grid, block, 0, s, P.tab, P.off, P.nj);
+}
+
+template <int SCH, int RIE, int R, typename T>
+void launch_sweep_pack_rt(const PackLaunch &P, hipStream_t s)
+{
+    if constexpr (edge_scheme<SCH, R, T>()) {
+        // each member in the form in which it runs alone: a launch for each form
+        PackLaunch a = P, b = P;
+        a.nj = P.nj_one; a.nblocks = P.nblocks_one;
+        b.tab += P.nj_one; b.off += P.nj_one; b.nj -= P.nj_one; b.nblocks -= P.nblocks_one;
+        if (a.nj > 0) launch_sweep_pack_rte<SCH, RIE, R, T, EDGE_AHEAD>(a, s);
+        if (b.nj > 0) launch_sweep_pack_rte<SCH, RIE, R, T, EDGE_IN_LOOP>(b, s);
+    } else {
+        launch_sweep_pack_rte<SCH, RIE, R, T, EDGE_IN_LOOP>(P, s);
+    }
 }
 
 template <int SCH, int RIE, int R>

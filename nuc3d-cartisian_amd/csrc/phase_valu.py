@@ -9,7 +9,7 @@ computes:
   splitting) are constants, so that every block is executed exactly once per
   wave and the static count of each phase is its dynamic count per wave;
 - an empty asm statement with a scheduling barrier marks each phase boundary;
-- inside a CRWENO5 row the indicator, weight and row values pass through empty
+- inside a CRWENO5 row (FP64) the indicator and weight values pass through empty
   asm statements, so that the compiler cannot move their arithmetic across the
   boundaries.
 
@@ -50,39 +50,32 @@ SWEEP_EDITS = [
     ("#pragma unroll 1\n    for (int v = 0; v < 5; v++) {",
      "#pragma unroll\n    for (int v = 0; v < 5; v++) {\n        PH(split);"),
     ("    // split parameters of the own cells", "    PH(prologue);\n    // split parameters of the own cells"),
-    ("        fetch(v + 1, qnx, xnx);", "        PH(fetch);\n        fetch(v + 1, qnx, xnx);"),
-    ("        sync_lines(d);\n        double out[R];", "        PH(barrier);\n        sync_lines(d);\n        double out[R];"),
+    ("        if constexpr (F::PREF) fetch(v + 1, qnx, xnx);", "        PH(fetch);\n        if constexpr (F::PREF) fetch(v + 1, qnx, xnx);"),
+    ("        sync_lines<WPL>(d);\n        double out[R];", "        PH(barrier);\n        sync_lines<WPL>(d);\n        double out[R];"),
     ("        sync_wave();\n        if (wv) {", "        PH(write_interfaces);\n        sync_wave();\n        if (wv) {"),
+    ("        if constexpr (!F::PREF) fetch(v + 1, qnx, xnx);", "        PH(fetch);\n        if constexpr (!F::PREF) fetch(v + 1, qnx, xnx);"),
     ("        // the final phase's own global reads", "        PH(final);\n        // the final phase's own global reads"),
 ]
 LINES_EDITS = [
-    ("    T win[W];\n#pragma unroll\n    for (int t = 0; t < W; t++) win[t]",
-     "    PH(window);\n    T win[W];\n#pragma unroll\n    for (int t = 0; t < W; t++) win[t]"),
-    ("            T f4 = win[r + 4];\n            T d4 = f4 - f3;\n            T e3 = T(13.0 / 12.0) * sq(d4 - d3);\n"
-     "            T b0, b1, b2, q0, q1, q2, h2;\n            w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);\n"
-     "            TW P0, P1, P2;",
-     "            PH(indicators);\n            T f4 = win[r + 4];\n            T d4 = f4 - f3;\n            T e3 = T(13.0 / 12.0) * sq(d4 - d3);\n"
-     "            T b0, b1, b2, q0, q1, q2, h2;\n            w5_diff<T>(f2, f3, d1, d2, d3, d4, e1, e2, e3, b0, b1, b2, q0, q1, q2, h2);\n"
-     "            TW P0, P1, P2;"),
-    ("            TW P0, P1, P2;   // weights with unit ideal weights\n"
-     "            w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);\n"
-     "            // Every row is scaled",
-     "            asm volatile(\"\" : \"+v\"(b0), \"+v\"(b1), \"+v\"(b2), \"+v\"(q0), \"+v\"(q1), \"+v\"(q2));\n"
-     "            PH(weights);\n"
-     "            TW P0, P1, P2;   // weights with unit ideal weights\n"
-     "            w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);\n"
-     "            asm volatile(\"\" : \"+v\"(P0), \"+v\"(P1), \"+v\"(P2));\n"
-     "            PH(rows);\n"
-     "            // Every row is scaled"),
-    ("                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            ch.row(r, a, b, c, d);",
-     "                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            PH(elimination);\n"
-     "            ch.row(r, a, b, c, d);"),
-    ("        ch.solve(h);\n#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n    } else if constexpr (SCH == HCCS77)",
-     "        PH(back_substitution);\n        ch.solve(h);\n#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n"
-     "    } else if constexpr (SCH == HCCS77)"),
-    ("        pcr32(al, ga, de, h);\n        T X1 = de;", "        PH(pcr);\n        pcr32(al, ga, de, h);\n        PH(fold_back);\n        T X1 = de;"),
+    ("        constexpr bool AHEAD = EDGE == EDGE_AHEAD;\n", "        constexpr bool AHEAD = EDGE == EDGE_AHEAD;\n        PH(explicit_rows);\n"),
+    ("            asm volatile(\"; explicit rows ahead\" ::: \"memory\");\n", "            PH(window);\n"),
+    ("            T f4 = win[O + r + 4];\n", "            PH(indicators);\n            T f4 = win[O + r + 4];\n"),
+    ("                w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);\n                if constexpr (!AHEAD)",
+     "                asm volatile(\"\" : \"+v\"(b0), \"+v\"(b1), \"+v\"(b2));\n"
+     "                PH(weights);\n"
+     "                w5_weights<TW>(TW(b0), TW(b1), TW(b2), TW(1), TW(1), TW(1), P0, P1, P2);\n"
+     "                asm volatile(\"\" : \"+v\"(P0), \"+v\"(P1), \"+v\"(P2));\n"
+     "                PH(rows);\n"
+     "                if constexpr (!AHEAD)"),
+    ("                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            ch.row(r, a, b, c, d);\n"
+     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        ch.solve(h);\n"
+     "#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n    } else if constexpr (SCH == HCCS77) {",
+     "                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            PH(elimination);\n            ch.row(r, a, b, c, d);\n"
+     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        PH(back_substitution);\n        ch.solve(h);\n"
+     "#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n    } else if constexpr (SCH == HCCS77) {"),
+    ("        pcr<NL, F32>(al, ga, de);\n        T X1 = de;", "        PH(pcr);\n        pcr<NL, F32>(al, ga, de);\n        PH(fold_back);\n        T X1 = de;"),
 ]
-ORDER = ["entry", "prologue", "split", "fetch", "barrier", "window", "indicators", "weights", "rows",
+ORDER = ["entry", "prologue", "split", "fetch", "barrier", "explicit_rows", "window", "indicators", "weights", "rows",
          "elimination", "back_substitution", "pcr", "fold_back", "write_interfaces", "final"]
 
 
@@ -147,8 +140,9 @@ def count(asm):
 
 def main():
     ap = argparse.ArgumentParser()
-    ap.add_argument("--inst", default="3, 0, 8, 4, double, true, 0",
-                    help="k_sweep template arguments (default: CRWENO5, LF, R=8, 4 lines, FP64, FULL, no RK3 update)")
+    ap.add_argument("--inst", default="3, 0, 8, 4, double, true, 0, double, false, 1, 1",
+                    help="k_sweep template arguments (default: CRWENO5, LF, R=8, 4 lines, FP64, FULL, no RK3 update, "
+                         "one wave a line, one-block lines)")
     ap.add_argument("--measured", type=float, default=None, help="measured VALU wave-instructions per wave")
     a = ap.parse_args()
     with tempfile.TemporaryDirectory() as tmp:

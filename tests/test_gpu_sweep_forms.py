@@ -34,6 +34,16 @@ CASES = [
     ((512, 10, 11), (1, 1, 1), G.HCCS, G.CD6, G.LF),
     ((12, 10, 512), (1, 1, 4), G.CRWENO5, G.CD8, G.LF),
     ((1022, 10, 11), (2, 1, 1), G.CRWENO5, G.CD6, G.LF),
+    # compact lines of one block (explicit rows ahead of the row loop): the
+    # shortest and longest line of each row count, with and without tails
+    ((65, 96, 97), (1, 1, 1), G.CRWENO5, G.CD6, G.AUSM),
+    ((65, 96, 97), (1, 1, 1), G.HCCS, G.CD8, G.LF),
+    ((128, 12, 160), (1, 1, 1), G.CRWENO5, G.CD8, G.LF),
+    ((129, 128, 12), (1, 1, 1), G.HCCS, G.CD6, G.AUSMP),
+    ((12, 161, 192), (1, 1, 1), G.CRWENO5, G.CD6, G.AUSMP),
+    ((192, 12, 193), (1, 1, 1), G.HCCS, G.CD6, G.LF),
+    ((193, 256, 12), (1, 1, 1), G.CRWENO5, G.CD8, G.LF),
+    ((256, 12, 193), (1, 1, 1), G.HCCS, G.CD8, G.AUSM),
 ]
 
 
@@ -71,3 +81,32 @@ def test_rhs_matches_oracle(case):
     print("rel err", err, "tol", tol, flush=True)
     assert np.all(err <= tol), (err, tol)
     assert abs(dt - dt_ref) <= 1e-14 * dt_ref
+
+
+@pytest.mark.parametrize("scheme,precision", [(G.CRWENO5, G.FP64), (G.CRWENO5, G.MIXED), (G.HCCS, G.FP64)])
+def test_pack_of_one_block_and_rank_grid(scheme, precision):
+    """A pack whose members' lines are one block in some and several in others:
+    each member bit for bit as it runs alone."""
+    boxes = [((72, 66, 80), (1, 1, 1)), ((96, 70, 68), (1, 2, 1)), ((66, 96, 72), (1, 1, 1))]
+    cfgs = [G.make_config(n=n, npr=npr, scheme=scheme, vis=G.CD6, riemann=G.LF, model=G.NAVIERSTOKES3D,
+                          precision=precision) for n, npr in boxes]
+    qs = [_state(O.make_config(n=n, npr=npr), 20 + k) for k, (n, npr) in enumerate(boxes)]
+    alone = []
+    for c, q in zip(cfgs, qs):
+        with G.Context(c) as ctx:
+            ctx.upload(q)
+            ctx.step(2)
+            alone.append(ctx.download())
+    for members in ([0, 1, 2], [0, 2]):
+        ctxs = [G.Context(cfgs[k]) for k in members]
+        for ctx, k in zip(ctxs, members):
+            ctx.upload(qs[k])
+        with G.Pack(ctxs) as p:
+            p.step_async(2)
+            for ctx in ctxs:
+                ctx.sync()
+            got = [ctx.download() for ctx in ctxs]
+        for ctx in ctxs:
+            ctx.close()
+        for k, g in zip(members, got):
+            assert np.array_equal(g, alone[k]), (members, boxes[k])
