@@ -56,8 +56,9 @@ template <int SCH> struct Radius {
 template <int SCH> struct Extra { static constexpr int value = (SCH == HCCS78) ? 1 : 0; };
 
 // Skewed LDS line layout: position y (y >= -B) lives at slot (y+B) + (y+B)/R,
-// one pad slot after every R positions, B = HALO+1 rounded up to a multiple of
-// R.  The f^+ line stores cell x at y = x; the f^- line is stored mirrored,
+// one pad slot after every R positions, B = HALO+2 rounded up to a multiple of
+// R (the lowest position is that of the mirrored write-only dummy, cell NL R+HALO,
+// y = -(HALO+2)).  The f^+ line stores cell x at y = x; the f^- line is stored mirrored,
 // y = NL R-2-x (NL lanes per sign), so that both signs read their windows upwards from
 // y = hR-RAD-1: the lane's window then starts at slot h*(R+1) + at(-RAD-1)
 // and every window element is a compile-time offset from one base.  Lanes R
@@ -67,9 +68,9 @@ template <int SCH> struct Extra { static constexpr int value = (SCH == HCCS78) ?
 // lines x 4 consecutive cells per 16 lanes, which then hit distinct banks
 // (measured: y/z sweep bank-conflict cycles -79% against a pitch = 2 mod 16).
 template <int R, int NL = 32> struct Skew {
-    static constexpr int B = ((HALO + 1 + R - 1) / R) * R;
+    static constexpr int B = ((HALO + 2 + R - 1) / R) * R;
     __host__ __device__ static constexpr int at(int y) { return (y + B) + (y + B) / R; }
-    __device__ __forceinline__ static int mir(int x) { return at(NL * R - 2 - x); }
+    __host__ __device__ static constexpr int mir(int x) { return at(NL * R - 2 - x); }
     // slots up to cell ncap+HALO: the last one is a write-only dummy (halo
     // writes of interior cells go there instead of branching)
     static constexpr int span(int ncap) { return at(ncap + HALO) + 1; }
