@@ -1,0 +1,81 @@
+// nuc_transfer.hip over a HIP runtime on the host (host_hip): what its copies
+// promise about the bytes, the threads beside them and the calling thread.
+#include "nuc_transfer.hip"
+
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <future>
+#include <string>
+
+static int failed = 0;
+#define CHECK(c, ...) do { if (!(c)) { failed++; std::printf("line %d: %s: ", __LINE__, #c); std::printf(__VA_ARGS__); std::printf("\n"); } } while (0)
+
+static std::vector<double> values(size_t n, unsigned seed)
+{
+    std::vector<double> v(n);
+    uint64_t x = seed * 2654435761u + 1;
+    for (double &d : v) { x = x * 6364136223846793005ull + 1442695040888963407ull; d = double(x >> 11); }
+    return v;
+}
+
+// past the bytes from which the staging memory is pinned
+static void warm(hosthip::Stream &s)
+{
+    std::vector<double> a(size_t(9) << 20), d(a.size());
+    nuctransfer::copy(d.data(), a.data(), 8 * a.size(), hipMemcpyHostToDevice, &s);
+    hosthip::staged_kernels = hosthip::plain_copies = hosthip::pinned_copies = 0;
+}
+
+// Bytes both ways at sizes around the limits and the chunks; `off` values of the
+// device array are skipped, so that its chunks begin 8 bytes off 16
+static void bytes()
+{
+    hosthip::Stream s(0);
+    nuctransfer::retain();
+    warm(s);
+    const size_t MB = size_t(1) << 20;
+    const size_t sizes[] = {8 * MB - 8, 8 * MB, 8 * MB + 8, 16 * MB - 8, 16 * MB, 16 * MB + 8, 20 * MB, 32 * MB,
+                            32 * MB + 8, 36 * MB - 16, 64 * MB + 24, 69 * MB + 8};
+    for (size_t n8 : sizes)
+        for (size_t off : {0, 1}) {
+            const size_t n = n8 / 8;
+            std::vector<double> h = values(n, unsigned(n + off)), d(n + off + 2, -1.0), back(n + 2, -2.0);
+            hosthip::staged_kernels = hosthip::plain_copies = hosthip::pinned_copies = 0;
+            CHECK(nuctransfer::copy(d.data() + off, h.data(), n8, hipMemcpyHostToDevice, &s) == hipSuccess, "up");
+            CHECK(std::memcmp(d.data() + off, h.data(), n8) == 0 && d[n + off] == -1.0, "%zu bytes up", n8);
+            CHECK((hosthip::pinned_copies > 0) == (n8 >= 16 * MB), "%zu bytes up: %d staged", n8, hosthip::pinned_copies);
+            for (size_t i = 0; i < n; i++) h[i] = d[off + i] = h[i] + 1.0;   // other bytes than the slots still hold
+            CHECK(nuctransfer::copy(back.data(), d.data() + off, n8, hipMemcpyDeviceToHost, &s) == hipSuccess, "down");
+            CHECK(std::memcmp(back.data(), h.data(), n8) == 0 && back[n] == -2.0, "%zu bytes down, offset %zu", n8, off);
+            CHECK((hosthip::staged_kernels > 0) == (n8 >= 8 * MB), "%zu bytes down: %d staged", n8, hosthip::staged_kernels);
+        }
+    // memory the runtime knows, and sizes that are no whole number of doubles, are not staged
+    void *p = nullptr;
+    CHECK(hipHostMalloc(&p, 32 * MB, hipHostMallocDefault) == hipSuccess, "pinned");
+    std::vector<double> d(4 * MB);
+    hosthip::staged_kernels = hosthip::plain_copies = hosthip::pinned_copies = 0;
+    CHECK(nuctransfer::copy(p, d.data(), 32 * MB, hipMemcpyDeviceToHost, &s) == hipSuccess, "down");
+    CHECK(hosthip::staged_kernels == 0 && hosthip::pinned_copies == 1, "a pinned array is copied as it is");
+    std::vector<char> odd(32 * MB);
+    CHECK(nuctransfer::copy(odd.data(), d.data(), 32 * MB - 3, hipMemcpyDeviceToHost, &s) == hipSuccess, "down");
+    CHECK(hosthip::staged_kernels == 0 && hosthip::plain_copies == 1, "%d", hosthip::staged_kernels);
+    hipHostFree(p);
+    nuctransfer::release();
+    CHECK(hosthip::pinned.empty(), "the staging memory is given back");
+    // where no memory can be pinned the runtime copies
+    nuctransfer::retain();
+    hosthip::refuse_pinned = 1;
+    std::vector<double> h = values(size_t(10) * MB, 7), e(h.size());
+    CHECK(nuctransfer::copy(e.data(), h.data(), 8 * h.size(), hipMemcpyHostToDevice, &s) == hipSuccess && e == h, "refused");
+    hosthip::refuse_pinned = 0;
+    nuctransfer::release();
+}
+
+int main(int argc, char **argv)
+{
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "bytes") bytes();
+    else { std::printf("unknown case\n"); return 2; }
+    return failed != 0;
+}
