@@ -18,6 +18,7 @@
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <utility>
 
 namespace nuctransfer {
 namespace {
@@ -30,14 +31,19 @@ constexpr int OUT_BLOCKS = 16;         // fill the link (16 to 256 measured alik
 // down 0.79 against 0.63; 35 MB up 1.14 against 0.94).
 constexpr size_t MIN_UP = size_t(16) << 20, MIN_DOWN = size_t(8) << 20;
 
-std::mutex g_mu;                       // the staging memory and its user count
+std::mutex g_users_mu;                 // the user count
+int g_users = 0;
+// The staging memory and what follows.  Held while a copy is staged, but neither
+// by callers that only come or go nor while a copy waits for its stream's earlier
+// work, so that contexts are created and destroyed, and others copy, beside one
+// that downloads behind queued steps.  Taken after g_users_mu where both are.
+std::mutex g_stage_mu;
 // 2 * THREADS slots of CHUNK bytes (64 MiB), pinned.  Coherent: a worker reads a
 // slot once the event behind its kernel is reached, and only coherent memory is
 // promised to show a kernel's stores by then (other pinned memory: after a
 // release at system scope, which an event need not be).  As fast: 256^3 down
 // 14.8 and 14.7 ms, up 14.6 and 14.5.
 char *g_stage = nullptr;
-int g_users = 0;
 size_t g_seen = 0;                     // bytes that would have been staged since the memory was last given back
 
 // A chunk into a pinned slot by stores over the link.  hipMemcpyAsync down
@@ -115,8 +121,10 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
     const bool up = kind == hipMemcpyHostToDevice;
     const void *host = up ? src : dst;
     if (bytes >= (up ? MIN_UP : MIN_DOWN) && bytes % 8 == 0 && !known(host)) {
+        const hipError_t earlier = hipStreamSynchronize(s);   // before the staging memory is taken
+        if (earlier != hipSuccess) return earlier;
         // one staged copy at a time; another thread's takes the plain path meanwhile
-        std::unique_lock<std::mutex> lk(g_mu, std::try_to_lock);
+        std::unique_lock<std::mutex> lk(g_stage_mu, std::try_to_lock);
         if (lk.owns_lock()) {
             // pinning it takes about 4 ms: only once the arrays have made up for that
             g_seen += bytes;
@@ -153,18 +161,22 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
 
 void retain()
 {
-    std::lock_guard<std::mutex> lk(g_mu);
+    std::lock_guard<std::mutex> lk(g_users_mu);
     g_users++;
 }
 
 void release()
 {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (--g_users == 0) {
-        if (g_stage) (void)hipHostFree(g_stage);
-        g_stage = nullptr;
-        g_seen = 0;
+    char *gone = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(g_users_mu);
+        if (--g_users == 0) {
+            std::lock_guard<std::mutex> st(g_stage_mu);   // free: no user is left to copy
+            std::swap(gone, g_stage);
+            g_seen = 0;
+        }
     }
+    if (gone) (void)hipHostFree(gone);
 }
 
 }  // namespace nuctransfer

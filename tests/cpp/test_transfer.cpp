@@ -72,10 +72,41 @@ static void bytes()
     nuctransfer::release();
 }
 
+// A copy behind a stream's earlier work: contexts and serving loops come and go
+// meanwhile, and another stream's copy is staged
+static void locks()
+{
+    hosthip::Stream a(0), b(0);
+    nuctransfer::retain();
+    warm(a);
+    std::promise<void> gate;
+    std::shared_future<void> open = gate.get_future().share();
+    a.put([open] { open.wait(); });
+    std::vector<double> da = values(size_t(5) << 20, 1), db = values(size_t(5) << 20, 2), ha(da.size()), hb(db.size());
+    std::thread ta([&] { nuctransfer::copy(ha.data(), da.data(), 8 * da.size(), hipMemcpyDeviceToHost, &a); });
+    std::this_thread::sleep_for(std::chrono::milliseconds(200));   // into its copy
+    auto wait = [](std::future<void> &f) { return f.wait_for(std::chrono::seconds(10)) == std::future_status::ready; };
+    std::future<void> user = std::async(std::launch::async, [] { nuctransfer::retain(); nuctransfer::release(); });
+    CHECK(wait(user), "retain and release wait for another stream's work");
+    std::future<void> other = std::async(std::launch::async, [&] {
+        nuctransfer::copy(hb.data(), db.data(), 8 * db.size(), hipMemcpyDeviceToHost, &b);
+    });
+    CHECK(wait(other), "a copy waits for another stream's work");
+    CHECK(hosthip::staged_kernels > 0, "the copy beside a waiting one is not staged");
+    gate.set_value();
+    ta.join();
+    user.get();
+    other.get();
+    CHECK(ha == da && hb == db, "bytes");
+    nuctransfer::release();
+    CHECK(hosthip::pinned.empty(), "the staging memory is given back");
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") bytes();
+    else if (what == "locks") locks();
     else { std::printf("unknown case\n"); return 2; }
     return failed != 0;
 }
