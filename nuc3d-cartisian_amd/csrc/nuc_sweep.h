@@ -632,10 +632,16 @@ void launch_sweep_rtle(const SweepArgs &A, hipStream_t s)
 
 // CRWENO5 and hccs lines of one block evaluate their explicit rows ahead
 // (line_half); a line of several blocks (from four on they are more than a wave
-// has lanes) forms them in the row loop.  With two rows a lane the loop has two
-// rows to save on and pays one ahead; FP32 stencils save half as much and gained
-// nothing (256^3 mixed 644/745/760 us ahead, 648/744/759 in place).
-template <int SCH, int R, typename T> constexpr bool edge_scheme() { return (SCH == CRWENO5 || SCH == HCCS) && R > 2 && sizeof(T) == 8; }
+// has lanes) forms them in the row loop.  With few rows a lane the loop has few
+// to save on and pays one ahead: CRWENO5 begins at four rows (x/y/z us of 96^3
+// LF on three: 81.5/80.4/79.1 ahead, 77.2/76.8/75.2 in place; 96 and 90 cells in
+// larger boxes 3-5 % for either splitting), hccs, whose explicit row is longer,
+// at three.  FP32 stencils save half as much and gained nothing (256^3 mixed
+// 644/745/760 us ahead, 648/744/759 in place).
+template <int SCH, int R, typename T> constexpr bool edge_scheme()
+{
+    return ((SCH == CRWENO5 && R > 3) || (SCH == HCCS && R > 2)) && sizeof(T) == 8;
+}
 template <int SCH, int RIE, int R, int WPL, int LPB, bool SEG, typename T, typename S>
 void launch_sweep_rtl(const SweepArgs &A, hipStream_t s)
 {
