@@ -269,12 +269,18 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     int ll, g;
     if (d == 0) { ll = t / GS; g = t % GS; }
     else { ll = t % LPB; g = t / LPB; }
-    const long L = blk * LPB + ll;   // SEG: the segment L % nseg of line L / nseg
+    // SEG, x: a line's segments follow each other.  y and z: the lines of one
+    // segment do, so that a workgroup's are neighbours in x as whole lines are; with
+    // a line's segments side by side, two lines a workgroup read 8 contiguous bytes
+    // a cell (64x64x1022 z, us: CRWENO5/AUSM 688 -> 355, hccs/AUSM 694 -> 555;
+    // 64x64x1024 WENO5-JS on one wave a line 731 -> 276)
+    auto seg_of = [&](long l) { return (int)(d == 0 ? l % A.nseg : l / A.nlines); };
+    const long L = blk * LPB + ll;
     const long nll = SEG ? A.nlines * A.nseg : A.nlines;
     const bool lv = FULL || L < nll;
     long line = L;
     int seg = 0;
-    if constexpr (SEG) { line = L / A.nseg; seg = (int)(L - line * A.nseg); }
+    if constexpr (SEG) { seg = seg_of(L); line = d == 0 ? L / A.nseg : L - (long)seg * A.nlines; }
     long base = 0, stride = 1;
     if (d == 0) { base = line * A.nx; stride = 1; }
     else if (d == 1) { long i = line % A.nx, k = line / A.nx; base = i + (long)A.nx * A.ny * k; stride = A.nx; }
@@ -355,7 +361,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     const bool wv = FULL || blk * LPB + lw < nll;
     // the zones of the line this wave reconstructs (line `lw` of the
     // workgroup; in the y/z sweeps not the line of the thread's own cells)
-    const int offw = SEG ? (int)((blk * LPB + lw) % A.nseg) * n : 0;
+    const int offw = SEG ? seg_of(blk * LPB + lw) * n : 0;
     const Zone z{SEG ? n + 1 : n, A.nloc, A.ts, offw};
     // line-buffer slots of the thread's cells c = g + GS k and of c + 1 (f^+
     // skewed, f^- mirrored).  When R divides GS they are affine in k (the
