@@ -134,8 +134,8 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
                 g_stage = nullptr;
                 (void)hipGetLastError();
             }
-            int device = 0;
-            if (g_stage && hipStreamGetDevice(s, &device) == hipSuccess) {
+            int device = 0, callers = 0;
+            if (g_stage && hipStreamGetDevice(s, &device) == hipSuccess && hipGetDevice(&callers) == hipSuccess) {
                 std::atomic<int> err{hipSuccess};
                 char *h = static_cast<char *>(const_cast<void *>(host)), *d = static_cast<char *>(up ? dst : const_cast<void *>(src));
                 std::thread th[THREADS];
@@ -149,6 +149,7 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
                 work(0, h, d, bytes, up, s, device, &err);
                 for (int w = started + 1; w < THREADS; w++) work(w, h, d, bytes, up, s, device, &err);
                 for (int i = 0; i < started; i++) th[i].join();
+                if (callers != device) (void)hipSetDevice(callers);   // work() has set the stream's
                 // the slots are free for the next copy only when every copy has left them
                 const hipError_t e = hipStreamSynchronize(s);
                 return err.load() != hipSuccess ? (hipError_t)err.load() : e;

@@ -102,11 +102,29 @@ static void locks()
     CHECK(hosthip::pinned.empty(), "the staging memory is given back");
 }
 
+// The calling thread's current device is its own
+static void device()
+{
+    hosthip::Stream s(1);
+    nuctransfer::retain();
+    warm(s);
+    std::vector<double> h = values(size_t(5) << 20, 3), d(h.size()), r(h.size());
+    hosthip::device = 0;
+    nuctransfer::copy(d.data(), h.data(), 8 * h.size(), hipMemcpyHostToDevice, &s);
+    CHECK(hosthip::device == 0, "device %d after a copy up", hosthip::device);
+    hosthip::device = 0;
+    nuctransfer::copy(r.data(), d.data(), 8 * d.size(), hipMemcpyDeviceToHost, &s);
+    CHECK(hosthip::device == 0, "device %d after a copy down", hosthip::device);
+    CHECK(r == h && hosthip::staged_kernels > 0 && hosthip::pinned_copies > 0, "bytes, staged");
+    nuctransfer::release();
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") bytes();
     else if (what == "locks") locks();
+    else if (what == "device") device();
     else { std::printf("unknown case\n"); return 2; }
     return failed != 0;
 }
