@@ -15,8 +15,8 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <utility>
 
@@ -143,8 +143,8 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
                 try {
                     for (; started < THREADS - 1; started++)
                         th[started] = std::thread(work, started + 1, h, d, bytes, up, s, device, &err);
-                } catch (const std::system_error &) {
-                    // no more threads: the calling one does the rest
+                } catch (const std::exception &) {
+                    // no more threads, or no memory to start one: the calling one does the rest
                 }
                 work(0, h, d, bytes, up, s, device, &err);
                 for (int w = started + 1; w < THREADS; w++) work(w, h, d, bytes, up, s, device, &err);

@@ -119,12 +119,40 @@ static void device()
     nuctransfer::release();
 }
 
+// While set, this thread's allocations outside the runtime fail (a worker
+// thread's start among them)
+static thread_local bool refuse_new = false;
+
+void *operator new(size_t n)
+{
+    if (refuse_new && !hosthip::inside) throw std::bad_alloc();
+    if (void *p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
+static void no_threads()
+{
+    hosthip::Stream s(0);
+    nuctransfer::retain();
+    warm(s);
+    std::vector<double> h = values((size_t(5) << 20) + 3, 4), d(h.size()), r(h.size());
+    refuse_new = true;
+    const hipError_t up = nuctransfer::copy(d.data(), h.data(), 8 * h.size(), hipMemcpyHostToDevice, &s);
+    const hipError_t down = nuctransfer::copy(r.data(), d.data(), 8 * d.size(), hipMemcpyDeviceToHost, &s);
+    refuse_new = false;
+    CHECK(up == hipSuccess && down == hipSuccess && r == h, "without memory for worker threads");
+    nuctransfer::release();
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") bytes();
     else if (what == "locks") locks();
     else if (what == "device") device();
+    else if (what == "no_threads") no_threads();
     else { std::printf("unknown case\n"); return 2; }
     return failed != 0;
 }
