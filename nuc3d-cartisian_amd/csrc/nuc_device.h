@@ -215,8 +215,8 @@ __device__ __forceinline__ TW weno3js(const T *f)
 // With S_k = (is_k + eps)^2 the unnormalised weights are c_k (S_k + tau^2)/S_k.
 // Their sum less 1 is X = tau^2 sum_k c_k prod_{j!=k} S_j / (S_0 S_1 S_2),
 // theta = 1/(1 + X^2) and the CRWENO row's factor (1 - theta)/theta = X^2:
-// two reciprocals in place of seven quotients.  The products hold indicators
-// between 1e-40 and 1e50 (fluxes up to about 1e25).
+// two reciprocals in place of seven quotients.  X^2 holds fluxes up to about 1e17
+// beside indicators of zero, the products 1e22 (LineScale keeps them below 1e14).
 template <typename T, typename TW>
 __device__ __forceinline__ void hccs_row(T f0, T f1, T f2, T f3, T f4, T b0, T b1, T b2, TW &lo, TW &di, TW &hi, TW &rhs)
 {

@@ -277,6 +277,44 @@ __device__ __forceinline__ void w5_diff(T f2, T f3, T d1, T d2, T d3, T d4, T e1
     q2 = f3 - (T(1.0 / 3.0) * d3 + T(1.0 / 6.0) * d4);
 }
 
+// The Z-type schemes multiply squared indicators (WENO5-Z and hccs rows: the 12th
+// power of a flux, WENO7-Z the 4th) and hccs and its relatives square (tau/eps)^2
+// once more, which leaves FP64's range from fluxes of about 1e17 on.  Their
+// reconstruction scales with the line's values except for eps (1e-20, 1e-40), so a
+// wave that holds a value of 2^45 (3.5e13) or more forms its rows of the values
+// times a power of two that brings the largest there.  eps counts for more then,
+// but against values 1e30 times smaller than the line's largest only.
+// The test reads the values' high words as FP32 numbers, which order as the doubles
+// do (infinities and NaN are numbers to neither, and pass): one instruction for two
+// values, where a row has 75 to 210.  Rows formed twice, with a quotient for each
+// indicator the second time, cost registers instead: 5 % on average, hccs78 twice
+// the time in some forms; this is 0.6 %, at most 3 (kernels of hccs and WENO7).
+template <int SCH> constexpr bool z_type() { return SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78; }
+struct LineScale {
+    int k = 0;   // of the wave, in the place of a double's exponent
+    __device__ __forceinline__ double down() const { return __hiloint2double((1023 << 20) - k, 0); }
+    __device__ __forceinline__ double up() const { return __hiloint2double((1023 << 20) + k, 0); }
+    __device__ __forceinline__ bool on() const { return __builtin_expect(k != 0, 0); }
+    // looks at f[FROM .. FROM + COUNT), which hold every value of the line in some lane
+    template <int FROM, int COUNT, int N> __device__ __forceinline__ void apply(double (&f)[N])
+    {
+        float m = 0.f;
+#pragma unroll
+        for (int i = FROM; i < FROM + COUNT; i += 2)
+            asm("v_max3_f32 %0, %1, |%2|, |%3|"
+                : "=v"(m) : "v"(m), "v"(__double2hiint(f[i])), "v"(__double2hiint(f[i + 1 < FROM + COUNT ? i + 1 : i])));
+        constexpr int TOP = (1023 + 45) << 20;
+        if (__builtin_expect(__any(__float_as_int(m) >= TOP), 0)) {
+            // the exponent of the wave's largest value above 2^45, bit by bit
+#pragma unroll 1
+            for (int b = 512 << 20; b >= 1 << 20; b >>= 1)
+                if (__any(__float_as_int(m) >= TOP + k + b)) k += b;
+#pragma unroll
+            for (int i = 0; i < N; i++) f[i] *= down();
+        }
+    }
+};
+
 // The explicit rows of a compact line of one block (2 ts + 1 around interfaces
 // 0 and nloc, ts the scheme's own tilesize), numbered k = 0 .. 2 (2 ts + 1) - 1:
 // the interface m of row k; its place in row order is m of f^+, NL R - 1 - m of f^-.
@@ -312,17 +350,22 @@ template <int SCH> __device__ __forceinline__ bool edge_mine(const Zone &z, int 
 // evaluated ahead.  They are then in slot edge_slot(k) of the wave's and sign's
 // line buffer Lx, and out[] of those rows is meaningless.
 // tails: rows past the line's last interface read defined (finite) cells.
+// PERIODIC: cells outside the lanes' own R positions are images of cells inside.
 enum { EDGE_IN_LOOP = 0, EDGE_AHEAD = 1 };
-template <int SCH, int R, typename T, typename TW, typename TS, int NL = 32, int EDGE = EDGE_IN_LOOP>
+template <int SCH, int R, typename T, typename TW, typename TS, int NL = 32, int EDGE = EDGE_IN_LOOP, bool PERIODIC = false>
 __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const Zone &z, int h, bool neg,
                                           TS out[R], bool full = false, TS *Lx = nullptr, bool tails = false)
 {
     constexpr int RAD = Radius<SCH>::value;
     constexpr int W = R + 2 * RAD + Extra<SCH>::value;
     T win[W];
+    constexpr bool SCALED = z_type<SCH>() && sizeof(T) == 8;
+    constexpr int LOOK = PERIODIC ? RAD + 1 : 0, LOOKS = PERIODIC ? R : W;   // LineScale
+    LineScale sc;
     if constexpr (EDGE == EDGE_IN_LOOP) {
 #pragma unroll
         for (int t = 0; t < W; t++) win[t] = Lw[Skew<R>::at(t - RAD - 1)];
+        if constexpr (SCALED) sc.template apply<LOOK, LOOKS>(win);
     }
     // rank-local position of each row, without integer division in the loop
     int ml[R];
@@ -376,8 +419,8 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             // alpha_k = c_k (1 + (tau/s_k)^2), s_k = is_k + eps (src/weno5z.cpp:84-92),
             // scaled by s_0^2 s_1^2 s_2^2: no quotient is left but the normalisation
             // (three IEEE quotients are 35 of the plain form's 75 instructions).  The
-            // products hold indicators between eps = 1e-40 and 1e50.  FP32 stencils
-            // keep the plain form and its roundings (weno7z).
+            // products hold fluxes up to about 1e21 (LineScale keeps them below).  FP32
+            // stencils keep the plain form and its roundings (weno7z).
             const TW eps = TW(W5_FOUR<T> ? 4.0e-40 : 1.0e-40);
             const TW B0 = b0, B1 = b1, B2 = b2;
             TW a0, a1, a2;
@@ -517,6 +560,12 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         constexpr int O = RAD - RAD5;
         Chunk<R, TS, NL> ch;
         constexpr bool AHEAD = EDGE == EDGE_AHEAD;
+        auto scale_edges = [&](TS f) {   // the explicit rows' values with the line's
+            if (h < 2 * (2 * edge_ts<SCH>() + 1)) Lx[edge_slot<R, NL>(h)] *= f;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
         if constexpr (AHEAD) {
             const T *const Lb = Lw - h * (R + 1);
             const int m = edge_row<SCH>(z, h);
@@ -526,7 +575,10 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             for (int j = 0; j < 2 * RAD + 1; j++) fe[j] = Lb[Skew<R>::at(y - RAD - 1 + j)];
             TS x;
             if constexpr (SCH == HCCS) {
+                LineScale se;
+                if constexpr (SCALED) se.template apply<0, 2 * RAD + 1>(fe);
                 x = TS(weno7z<T, TW>(fe, TW(1.0e-40)));
+                if (se.on()) x *= se.up();
             } else {
                 const T c1 = fe[1] - fe[0], c2 = fe[2] - fe[1], c3 = fe[3] - fe[2], c4 = fe[4] - fe[3];
                 const T k1 = w5_g<T>() * sq(c2 - c1), k2 = w5_g<T>() * sq(c3 - c2), k3 = w5_g<T>() * sq(c4 - c3);
@@ -545,6 +597,10 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             asm volatile("; explicit rows ahead" ::: "memory");
 #pragma unroll
             for (int t = 0; t < W; t++) win[t] = Lw[Skew<R>::at(t - RAD - 1)];
+            if constexpr (SCALED) {
+                sc.template apply<LOOK, LOOKS>(win);
+                if (sc.on()) scale_edges(sc.down());
+            }
         }
         // rows in order, as above
         T f1 = win[O + 1], f2 = win[O + 2], f3 = win[O + 3];
@@ -627,6 +683,8 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
             ch.row(r, a, b, c, d);
             f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;
         }
+        if constexpr (AHEAD && SCALED)
+            if (sc.on()) scale_edges(sc.up());
         ch.solve(h);
 #pragma unroll
         for (int r = 0; r < R; r++) out[r] = ch.Df[r];
@@ -661,6 +719,12 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         ch.solve(h);
 #pragma unroll
         for (int r = 0; r < R; r++) out[r] = ch.Df[r];
+    }
+    if constexpr (SCALED) {
+        if (sc.on()) {
+#pragma unroll
+            for (int r = 0; r < R; r++) out[r] *= sc.up();
+        }
     }
 }
 

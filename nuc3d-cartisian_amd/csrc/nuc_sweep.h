@@ -385,11 +385,12 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
     const int mstep = neg ? -1 : 1;
     double res = 0.0;
     const double dt = epi ? *A.dtp : 0.0;
-    // The compact schemes' rows past the line's last interface: with FP64 line
-    // buffers the cells they read are set to zero here and never written again
-    // (the interface values stay below them), so that these rows are finite and
-    // need no replacement; the line's last row does not couple to them.
-    constexpr bool TAILS = F::COMPACT && !FULL && sizeof(T) == 8;
+    // Rows past the line's last interface: with FP64 line buffers the cells they
+    // read are set to zero here and never written again (the interface values stay
+    // below them).  The compact schemes' rows are then finite and need no
+    // replacement, as the line's last row does not couple to them; and the Z-type
+    // schemes find no value there that is not the line's (LineScale).
+    constexpr bool TAILS = (F::COMPACT || z_type<SCH>()) && !FULL && sizeof(T) == 8;
     if constexpr (TAILS) {
         for (int c = n + HALO + g; c <= NL * R + 2; c += GS) {
             Pl[Sk::at(c)] = T(0);
@@ -478,7 +479,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs &A, const long blk)
         // with eps down to 1e-40 and stay FP64
         constexpr bool zw = SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78;
         using TW = typename std::conditional<zw, double, T>::type;
-        if (wv) line_half<SCH, R, T, TW, double, NL, EDGE>(Lw, m0r, mstep, z, h, neg, out, FULL, neg ? Mw : Pw, TAILS);
+        if (wv) line_half<SCH, R, T, TW, double, NL, EDGE, !SEG>(Lw, m0r, mstep, z, h, neg, out, FULL, neg ? Mw : Pw, TAILS);
         // the interface values overwrite the wave's own line only: the
         // reconstruction of the other waves is not waited for
         sync_wave();
