@@ -211,29 +211,32 @@ __device__ __forceinline__ int wrapi(int i, int n) { return i < 0 ? i + n : (i >
 // gather kernel, and no primitive field round-trips through HBM.
 constexpr int GTX = 32, GTY = 16;
 // Planes per workgroup of the march: a workgroup costs its planes and about two
-// more for the queue's first eight, and one FP64 workgroup fills a CU, so the
-// march takes as many rounds of the 256 CUs as it has workgroups.  The least
+// more for the queue's first eight, and the march takes as many rounds of the 256
+// CUs as it has workgroups.  An FP64 workgroup fills a CU (183 registers); of those
+// with FP32 fluxes (124) two share one and take 1.35 times as long.  The least
 // rounds x (planes + 2), and of equals the longer march (fewer halo planes).
-// Measured (FP64, us, by planes 1 2 4 8 16 32): 32^3 6 9 15 27 - -; 64^3 16 12 16
-// 28 52 -; 96^3 62 55 41 34 54 -; 128^3 133 100 82 74 69 112; 256^3 1167 903 727
-// 639 599 581.
-inline int march_planes(int nx, int ny, int nz, int most)
+// Measured (us, by planes 1 2 4 8 16 32), FP64: 64^3 16 12 16 28 52 -; 96^3 62 55
+// 41 34 54 -; 128^3 133 100 82 74 69 112; 256^3 1167 903 727 639 599 581.  FP32 (as
+// it takes them, marches of idle CUs cut): 128^3 62 46 41 38 52 52; 205x210x64 103 79 70
+// 67 67 101; 192x192x64 76 61 54 59 63 59; 256^3 513 399 345 320 309 307.
+inline int march_planes(int nx, int ny, int nz, int most, bool f32)
 {
     const long tiles = (long)((nx + GTX - 1) / GTX) * ((ny + GTY - 1) / GTY);
     long best = 0;
     int planes = 1;
     for (int g = most; g >= 1; g = g > 32 ? 32 : g & (g - 1) ? g & (g - 1) : g / 2) {
-        const long rounds = (tiles * ((nz + g - 1) / g) + 255) / 256, cost = rounds * (g + 2);
+        const long rounds = (tiles * ((nz + g - 1) / g) + 255) / 256;
+        const long cost = (f32 ? rounds / 2 * 27 + rounds % 2 * 20 : rounds * 20) * (g + 2);
         if (best == 0 || cost < best) { best = cost; planes = g; }
     }
     return planes;
 }
-inline int grad_planes(int nx, int ny, int nz) { return march_planes(nx, ny, nz, nz < 32 ? nz : 32); }
+inline int grad_planes(int nx, int ny, int nz, bool f32) { return march_planes(nx, ny, nz, nz < 32 ? nz : 32, f32); }
 // the march of a tile shape of g planes: cut where it would leave CUs idle
-inline int cut_planes(int nx, int ny, int nz, int g)
+inline int cut_planes(int nx, int ny, int nz, int g, bool f32)
 {
     const long tiles = (long)((nx + GTX - 1) / GTX) * ((ny + GTY - 1) / GTY);
-    return tiles * ((nz + g - 1) / g) >= 256 ? g : march_planes(nx, ny, nz, g);
+    return tiles * ((nz + g - 1) / g) >= 256 ? g : march_planes(nx, ny, nz, g, f32);
 }
 
 // primitives u, v, w, T of one cell from its five conserved values
@@ -1175,7 +1178,8 @@ static void stage_args(nuc_ctx *x, int in, int stage, int outb, bool epilogue, S
         }
         G.law = c.viscosity; G.re = c.reynolds; G.mach = c.mach; G.pr = c.prandtl; G.gamma = c.gamma;
         G.tref = c.t_ref; G.tinf = c.t_inf;
-        G.gkz = x->gkz > 0 ? cut_planes(x->n[0], x->n[1], x->n[2], x->gkz) : grad_planes(x->n[0], x->n[1], x->n[2]);
+        G.gkz = x->gkz > 0 ? cut_planes(x->n[0], x->n[1], x->n[2], x->gkz, x->fv32)
+                           : grad_planes(x->n[0], x->n[1], x->n[2], x->fv32);
         sa.ggrid = dim3((x->n[0] + GTX - 1) / GTX, (x->n[1] + GTY - 1) / GTY, (x->n[2] + G.gkz - 1) / G.gkz);
         sa.do_grad = true;
     }
@@ -1398,12 +1402,12 @@ extern "C" int nuc_autotune(nuc_ctx *x)
     hipEvent_t e0, e1;
     NUC_CHECK(x, hipEventCreate(&e0));
     NUC_CHECK(x, hipEventCreate(&e1));
-    int best = grad_planes(x->n[0], x->n[1], x->n[2]);
+    int best = grad_planes(x->n[0], x->n[1], x->n[2], x->fv32);
     float best_ms = 1e30f;
     for (int gkz : {4, 8, 16, 32}) {
         if (gkz > x->n[2]) continue;
         GradArgs G = sa.grad;
-        G.gkz = cut_planes(x->n[0], x->n[1], x->n[2], gkz);
+        G.gkz = cut_planes(x->n[0], x->n[1], x->n[2], gkz, x->fv32);
         const dim3 grid(sa.ggrid.x, sa.ggrid.y, (x->n[2] + G.gkz - 1) / G.gkz);
         float tot = 0.f;
         for (int rep = 0; rep < 4; rep++) {
@@ -1441,7 +1445,7 @@ extern "C" int nuc_set_tile_shape(nuc_ctx *x, int planes)
 extern "C" int nuc_tile_shape(const nuc_ctx *x, int *grad_planes_out)
 {
     if (!x || !grad_planes_out) return NUC_EINVAL;
-    *grad_planes_out = x->gkz > 0 ? x->gkz : grad_planes(x->n[0], x->n[1], x->n[2]);
+    *grad_planes_out = x->gkz > 0 ? x->gkz : grad_planes(x->n[0], x->n[1], x->n[2], x->fv32);
     return NUC_OK;
 }
 
