@@ -68,11 +68,11 @@ LINES_EDITS = [
      "                PH(rows);\n"
      "                if constexpr (!AHEAD)"),
     ("                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            ch.row(r, a, b, c, d);\n"
-     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        ch.solve(h);\n"
-     "#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n    } else if constexpr (SCH == HCCS77) {",
+     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        if constexpr (AHEAD && SCALED)\n"
+     "            if (sc.on()) scale_edges(sc.up());\n        ch.solve(h);\n",
      "                              \"+v\"(a), \"+v\"(b), \"+v\"(c), \"+v\"(d));\n            PH(elimination);\n            ch.row(r, a, b, c, d);\n"
-     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        PH(back_substitution);\n        ch.solve(h);\n"
-     "#pragma unroll\n        for (int r = 0; r < R; r++) out[r] = ch.Df[r];\n    } else if constexpr (SCH == HCCS77) {"),
+     "            f1 = f2; f2 = f3; f3 = f4; d1 = d2; d2 = d3; d3 = d4; e1 = e2; e2 = e3;\n        }\n        if constexpr (AHEAD && SCALED)\n"
+     "            if (sc.on()) scale_edges(sc.up());\n        PH(back_substitution);\n        ch.solve(h);\n"),
     ("        pcr<NL, F32>(al, ga, de);\n        T X1 = de;", "        PH(pcr);\n        pcr<NL, F32>(al, ga, de);\n        PH(fold_back);\n        T X1 = de;"),
 ]
 ORDER = ["entry", "prologue", "split", "fetch", "barrier", "explicit_rows", "window", "indicators", "weights", "rows",
