@@ -1,12 +1,13 @@
 // nuc_lines.h -- per-line interface computation shared by the production
 // sweep kernels and the per-Field operator kernels.
 //
-// One wave owns one line held in LDS on [-HALO, 32R+HALO).  Lanes 0..31
-// reconstruct f^+ and lanes 32..63 reconstruct f^- (src/euler3d.cpp:334-387
-// does the two as separate sweeps).  Lane h of a half owns a chunk of R
-// consecutive interfaces; the f^- half takes the chunks in mirrored order
-// (lane h <-> chunk 31-h, rows reversed), which turns the f^- stencils and its
-// tridiagonal system into the same shape as f^+, so both halves execute one
+// A line is held in LDS on [-HALO, NL R+HALO), with NL lanes for each sign: one
+// wave owns it, lanes 0..31 reconstruct f^+ and lanes 32..63 f^- (NL = 32), or, for
+// FP64 lines of 257-512 cells, two waves, one per sign (NL = 64); the reference
+// does the two signs as separate sweeps (src/euler3d.cpp:334-387).  Lane h of a
+// sign owns a chunk of R consecutive interfaces; f^- takes the chunks in mirrored
+// order (lane h <-> chunk NL-1-h, rows reversed), which turns the f^- stencils and
+// its tridiagonal system into the same shape as f^+, so both signs execute one
 // instruction stream.
 //
 // Rank-local zones follow the reference's inner/boundary split per MPI block
@@ -553,8 +554,7 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // other row reads.
         // Measured with the shorter indicators and reciprocals of the same rows, us
         // x/y/z: CRWENO5/LF 192^3 367/412/414 -> 361/400/385, 256^3 818/903/885 ->
-        // 825/851/836 (the x sweep, which applies the update, spills 12 registers
-        // either way), with AUSM 914/968/950 -> 862/914/890; hccs/LF 256^3
+        // 825/851/836 (the x sweep, which applies the update, spills 6 registers), with AUSM 914/968/950 -> 862/914/890; hccs/LF 256^3
         // 1220/1212/1184 -> 1133/1130/1118.
         constexpr int RAD5 = 2;   // the 5-point stencil's window is win[O..]
         constexpr int O = RAD - RAD5;

@@ -77,7 +77,9 @@ struct SweepArgs {
 // lane + 64k of line t/64 (contiguous, coalesced); for y and z the LPB lines
 // of a workgroup are consecutive in x and thread t owns cells t/LPB + 64k of
 // line t%LPB, so each load instruction reads LPB consecutive doubles per cell.
-// Compute mapping: wave w owns line w (both signs, see nuc_lines.h).
+// Compute mapping: wave w owns line w (both signs, see nuc_lines.h).  With two
+// waves a line (WPL = 2, FP64 lines of 257-512 cells) the strides are 128 cells,
+// and waves 2l and 2l+1 own the signs of line l.
 // ---------------------------------------------------------------------------
 template <int RIE, typename T>
 __device__ __forceinline__ void split_params(const T q[5], int d, T gamma, T sp[5], bool ausmp = false)
@@ -174,9 +176,10 @@ __device__ __forceinline__ long xcd_block(unsigned p, unsigned nb)
     return (long)x * q + (x < rem ? x : rem) + i;
 }
 
-// Line-buffer synchronisation: in the x sweep every wave loads and computes
-// its own line, so a wave-level barrier suffices (LDS operations of one wave
-// complete in order); the y/z load mapping spreads a line over all waves.
+// Line-buffer synchronisation: in the x sweep with one wave a line every wave
+// loads and computes its own line, so a wave-level barrier suffices (LDS
+// operations of one wave complete in order); two waves share a line, and the y/z
+// load mapping spreads a line over all waves.
 __device__ __forceinline__ void sync_wave()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -207,10 +210,13 @@ __device__ __forceinline__ void sync_lines(int d)
 // their five parameters to LDS for a fourth wave (WENO5-Z 256^3 x 0.73 -> 0.67,
 // WENO7 160^3 x 0.354 -> 0.337).  Their 8-row form with tails needs 159
 // registers and stays at three waves (230^3 0.72 ms against 0.75 with one
-// parameter in LDS).  With FP32 stencils the explicit schemes keep their
-// parameters in registers, which are half as many (and where the parameters are
-// decides which products of the splitting are fused, whose FP32 roundings show
-// in the results).
+// parameter in LDS).  Below five rows the compiler's choice stays (R = 3 and 4: 94
+// to 109 registers, four waves; built for five, with 96, sweeps of CRWENO5 lines
+// of 83-128 cells went between -6 and +7 %, us: 97x60x83 LF x 53.7 -> 50.4, 128^3
+// LF y 133.9 -> 136.7, 120x90x128 AUSM x 115.5 -> 123.1).  With FP32 stencils the
+// explicit schemes keep their parameters in registers, which are half as many (and
+// where the parameters are decides which products of the splitting are fused,
+// whose FP32 roundings show in the results).
 template <int SCH, int RIE, int R, int LPB, typename T, int EPI, int WPL, int EDGE> struct SweepForm {
     static constexpr bool COMPACT = SCH == CRWENO5 || SCH == HCCS || SCH == HCCS77;
     static constexpr int NL = 32 * WPL;           // lanes per sign
@@ -610,8 +616,10 @@ constexpr bool compact_scheme(int sch) { return sch == CRWENO5 || sch == HCCS ||
 // waves (512x256^2 CRWENO5 1.98 ms a sweep against 2.60 with 4 lines, 512x128^2
 // WENO5-Z/AUSM 0.40 against 0.51).  y and z: 4, whose loads read 32 contiguous
 // bytes per cell (512x64x512 WENO5-JS z 0.86 ms against 1.26 with 2), but 2 for
-// hccs and hccs77, whose 130-169 registers leave room for one workgroup of 8
-// waves on a CU (512^3 hccs/AUSM z 15.2 ms against 16.4).
+// hccs, hccs77 and CRWENO5 with AUSM, whose 141-168 registers leave room for one
+// workgroup of 8 waves on a CU, two waves per SIMD, or three of 4 (512^3 hccs/AUSM
+// z 15.2 ms against 16.4; CRWENO5/AUSM 512^3 y 8.8 against 9.5, z 13.2 against
+// 13.0, 256x512x256 y 2.13 against 2.48, 128x128x512 z 0.60 against 0.63).
 constexpr int lpb2_yz(int sch, int rie) { return sch == HCCS || sch == HCCS77 || (sch == CRWENO5 && rie != RIE_LF) ? 2 : SWEEP_LPB; }
 constexpr int sweep_lpb(int wpl, int dir, int sch, int rie) { return wpl == 1 ? SWEEP_LPB : dir == 0 ? 2 : lpb2_yz(sch, rie); }
 

@@ -14,8 +14,8 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # n, rank grid, scheme, viscous scheme, splitting
-    # hccs explicit rows evaluated ahead of the row loop (up to 2 blocks a
-    # line) and inside it (3 and more); 10 cells is the shortest block
+    # hccs explicit rows inside the row loop (lines of several blocks, and of two
+    # rows a lane); 10 cells is the shortest block
     ((10, 20, 30), (1, 2, 3), G.HCCS, G.CD6, G.AUSM),
     ((30, 10, 20), (3, 1, 2), G.HCCS, G.CD8, G.LF),
     ((12, 66, 33), (1, 3, 3), G.HCCS, G.CD6, G.AUSMP),

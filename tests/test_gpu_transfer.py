@@ -12,10 +12,12 @@ import nuc3d_amd as G
 
 pytestmark = pytest.mark.gpu
 
+# (staged once 64 MiB have crossed, as in test_gpu_staged.py: here the runtime copies
+# all but the last, which is staged down)
 SIZES = [(58, 58, 58),      # 7.8 MB: below both limits
-         (61, 61, 59),      # 8.8 MB: staged down only
-         (75, 75, 75),      # 16.9 MB: staged both ways, an odd number of values
-         (128, 64, 64),     # exactly five chunks
+         (61, 61, 59),      # 8.8 MB: above the limit down
+         (75, 75, 75),      # 16.9 MB: above both, an odd number of values
+         (128, 64, 64),     # 21 MB: exactly five chunks
          (103, 97, 101)]    # 40 MB: more chunks than workers, odd
 
 
