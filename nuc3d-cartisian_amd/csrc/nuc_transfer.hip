@@ -31,6 +31,16 @@ constexpr int OUT_BLOCKS = 16;         // fill the link (16 to 256 measured alik
 // down 0.79 against 0.63; 35 MB up 1.14 against 0.94).
 constexpr size_t MIN_UP = size_t(16) << 20, MIN_DOWN = size_t(8) << 20;
 
+// What staging a copy saves, us, by the measurements above and (whole passes of
+// upload, step and download) 17 MB down 0.5 ms, 10 MB 0.2 ms.
+size_t saving(size_t bytes, bool up) { return (bytes >> 20) * (up ? 10 : bytes >= (size_t(32) << 20) ? 70 : 20); }
+// Pinning the staging memory and giving it back takes 6-7 ms: only once the copies
+// have lost twice that, which a 256^3 state does in its first way down and a 64^3
+// one in 65 passes.  Pinned at the first 64 MiB it made contexts that live for a few
+// copies slower than the runtime's own (96^3, created, stepped once and destroyed:
+// 8.4 -> 15.2 ms; 76^3 with four passes 11 -> 18).
+constexpr size_t PIN_AFTER = 13000;
+
 std::mutex g_users_mu;                 // the user count
 int g_users = 0;
 // The staging memory and what follows.  Held while a copy is staged, but neither
@@ -44,7 +54,7 @@ std::mutex g_stage_mu;
 // release at system scope, which an event need not be).  As fast: 256^3 down
 // 14.8 and 14.7 ms, up 14.6 and 14.5.
 char *g_stage = nullptr;
-size_t g_seen = 0;                     // bytes that would have been staged since the memory was last given back
+size_t g_lost = 0;                     // us that copies lost by not being staged since the memory was last given back
 
 // A chunk into a pinned slot by stores over the link.  hipMemcpyAsync down
 // followed by an event costs 130 us a copy here whatever its size (4 MiB
@@ -126,9 +136,8 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
         // one staged copy at a time; another thread's takes the plain path meanwhile
         std::unique_lock<std::mutex> lk(g_stage_mu, std::try_to_lock);
         if (lk.owns_lock()) {
-            // pinning it takes about 4 ms: only once the arrays have made up for that
-            g_seen += bytes;
-            if (!g_stage && g_seen >= 2 * THREADS * CHUNK &&
+            if (!g_stage) g_lost += saving(bytes, up);
+            if (!g_stage && g_lost >= PIN_AFTER &&
                 hipHostMalloc((void **)&g_stage, 2 * THREADS * CHUNK,
                               hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
                 g_stage = nullptr;
@@ -174,7 +183,7 @@ void release()
         if (--g_users == 0) {
             std::lock_guard<std::mutex> st(g_stage_mu);   // free: no user is left to copy
             std::swap(gone, g_stage);
-            g_seen = 0;
+            g_lost = 0;
         }
     }
     if (gone) (void)hipHostFree(gone);

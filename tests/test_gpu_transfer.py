@@ -12,8 +12,8 @@ import nuc3d_amd as G
 
 pytestmark = pytest.mark.gpu
 
-# (staged once 64 MiB have crossed, as in test_gpu_staged.py: here the runtime copies
-# all but the last, which is staged down)
+# (staged once copies have lost time without it, as in test_gpu_staged.py: here the
+# runtime copies)
 SIZES = [(58, 58, 58),      # 7.8 MB: below both limits
          (61, 61, 59),      # 8.8 MB: above the limit down
          (75, 75, 75),      # 16.9 MB: above both, an odd number of values

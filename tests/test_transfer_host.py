@@ -20,7 +20,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["bytes", "locks", "device", "no_threads"])
+@pytest.mark.parametrize("case", ["bytes", "pinning", "locks", "device", "no_threads"])
 def test_transfer(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
