@@ -34,12 +34,13 @@ constexpr size_t MIN_UP = size_t(16) << 20, MIN_DOWN = size_t(8) << 20;
 // What staging a copy saves, us, by the measurements above and (whole passes of
 // upload, step and download) 17 MB down 0.5 ms, 10 MB 0.2 ms.
 size_t saving(size_t bytes, bool up) { return (bytes >> 20) * (up ? 10 : bytes >= (size_t(32) << 20) ? 70 : 20); }
-// Pinning the staging memory and giving it back takes 6-7 ms: only once the copies
-// have lost twice that, which a 256^3 state does in its first way down and a 64^3
-// one in 65 passes.  Pinned at the first 64 MiB it made contexts that live for a few
-// copies slower than the runtime's own (96^3, created, stepped once and destroyed:
-// 8.4 -> 15.2 ms; 76^3 with four passes 11 -> 18).
-constexpr size_t PIN_AFTER = 13000;
+// Pinning a slot and giving it back takes 0.4-0.6 ms (all of them 6-10): as many as
+// the array has chunks are pinned, and only once the copies have lost more than their
+// price, which a 256^3 state does in its first way down, a 96^3 one in its third pass
+// and a 64^3 one (three slots) in its twelfth.  All pinned at the first 64 MiB they made
+// contexts that live for a few copies slower than the runtime's own (96^3, created,
+// stepped once and destroyed: 8.4 -> 15.2 ms; 76^3 with four passes 11 -> 18).
+constexpr size_t PIN_AFTER = 800;      // us a slot
 
 std::mutex g_users_mu;                 // the user count
 int g_users = 0;
@@ -48,13 +49,15 @@ int g_users = 0;
 // work, so that contexts are created and destroyed, and others copy, beside one
 // that downloads behind queued steps.  Taken after g_users_mu where both are.
 std::mutex g_stage_mu;
-// 2 * THREADS slots of CHUNK bytes (64 MiB), pinned.  Coherent: a worker reads a
-// slot once the event behind its kernel is reached, and only coherent memory is
-// promised to show a kernel's stores by then (other pinned memory: after a
-// release at system scope, which an event need not be).  As fast: 256^3 down
-// 14.8 and 14.7 ms, up 14.6 and 14.5.
-char *g_stage = nullptr;
-size_t g_lost = 0;                     // us that copies lost by not being staged since the memory was last given back
+// Slots of CHUNK bytes, the first g_slots of them pinned (all: 64 MiB), in g_blocks
+// blocks; worker w's are w and THREADS + w.  Coherent: a worker reads a slot once the
+// event behind its kernel is reached, and only coherent memory is promised to show
+// a kernel's stores by then (other pinned memory: after a release at system scope,
+// which an event need not be).  As fast: 256^3 down 14.8 and 14.7 ms, up 14.6 and
+// 14.5.
+char *g_slot[2 * THREADS], *g_block[2 * THREADS];
+int g_slots = 0, g_blocks = 0;
+size_t g_lost = 0;                     // us that copies lost by not being staged since slots were last pinned or given back
 
 // A chunk into a pinned slot by stores over the link.  hipMemcpyAsync down
 // followed by an event costs 130 us a copy here whatever its size (4 MiB
@@ -70,7 +73,7 @@ using v2d = __attribute__((ext_vector_type(2))) double;
 // one worker's chunks w, w + THREADS, ...; the first error stops the others
 void work(int w, char *host, char *dev, size_t bytes, bool up, hipStream_t s, int device, std::atomic<int> *err)
 {
-    char *const slot[2] = {g_stage + (2 * w) * CHUNK, g_stage + (2 * w + 1) * CHUNK};
+    char *const slot[2] = {g_slot[w], g_slot[THREADS + w]};
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipError_t e = hipSetDevice(device);
     for (int k = 0; k < 2 && e == hipSuccess; k++) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
@@ -110,6 +113,18 @@ void work(int w, char *host, char *dev, size_t bytes, bool up, hipStream_t s, in
         if (ev[i]) (void)hipEventDestroy(ev[i]);
 }
 
+// the first n slots pinned, the missing ones in one block (each by itself: twice the time)
+void pin(int n)
+{
+    char *block = nullptr;
+    if (hipHostMalloc((void **)&block, (n - g_slots) * CHUNK, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    g_block[g_blocks++] = block;
+    for (; g_slots < n; g_slots++, block += CHUNK) g_slot[g_slots] = block;
+}
+
 // whether the runtime knows the pointer (pinned, managed or device memory):
 // those are copied without staging
 bool known(const void *p)
@@ -136,15 +151,16 @@ hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hi
         // one staged copy at a time; another thread's takes the plain path meanwhile
         std::unique_lock<std::mutex> lk(g_stage_mu, std::try_to_lock);
         if (lk.owns_lock()) {
-            if (!g_stage) g_lost += saving(bytes, up);
-            if (!g_stage && g_lost >= PIN_AFTER &&
-                hipHostMalloc((void **)&g_stage, 2 * THREADS * CHUNK,
-                              hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
-                g_stage = nullptr;
-                (void)hipGetLastError();
+            const int need = (int)std::min<size_t>(2 * THREADS, (bytes + CHUNK - 1) / CHUNK);
+            if (g_slots < need) {
+                g_lost += saving(bytes, up);
+                if (g_lost >= PIN_AFTER * (need - g_slots)) {
+                    pin(need);
+                    g_lost = 0;
+                }
             }
             int device = 0, callers = 0;
-            if (g_stage && hipStreamGetDevice(s, &device) == hipSuccess && hipGetDevice(&callers) == hipSuccess) {
+            if (g_slots >= need && hipStreamGetDevice(s, &device) == hipSuccess && hipGetDevice(&callers) == hipSuccess) {
                 std::atomic<int> err{hipSuccess};
                 char *h = static_cast<char *>(const_cast<void *>(host)), *d = static_cast<char *>(up ? dst : const_cast<void *>(src));
                 std::thread th[THREADS];
@@ -177,16 +193,19 @@ void retain()
 
 void release()
 {
-    char *gone = nullptr;
+    char *gone[2 * THREADS];
+    int n = 0;
     {
         std::lock_guard<std::mutex> lk(g_users_mu);
         if (--g_users == 0) {
             std::lock_guard<std::mutex> st(g_stage_mu);   // free: no user is left to copy
-            std::swap(gone, g_stage);
+            std::swap(n, g_blocks);
+            std::copy(g_block, g_block + n, gone);
+            g_slots = 0;
             g_lost = 0;
         }
     }
-    if (gone) (void)hipHostFree(gone);
+    for (int i = 0; i < n; i++) (void)hipHostFree(gone[i]);
 }
 
 }  // namespace nuctransfer

@@ -67,36 +67,45 @@ static void bytes()
     nuctransfer::retain();
     hosthip::refuse_pinned = 1;
     std::vector<double> h = values(size_t(10) * MB, 7), e(h.size());
-    CHECK(nuctransfer::copy(e.data(), h.data(), 8 * h.size(), hipMemcpyHostToDevice, &s) == hipSuccess && e == h, "refused");
+    for (int i = 0; i < 4; i++)
+        CHECK(nuctransfer::copy(e.data(), h.data(), 8 * h.size(), hipMemcpyDeviceToHost, &s) == hipSuccess && e == h, "refused");
+    CHECK(hosthip::pinned.empty(), "refused");
     hosthip::refuse_pinned = 0;
     nuctransfer::release();
 }
 
-// Pinning pays after copies that lose about 13 ms without it: a 671 MB array's way
-// down, but not the few copies of a short-lived context, whose sum starts again with
-// the next one
+// Slots are pinned once copies have lost 0.8 ms for each that the array needs: on a
+// 704 MB array's way down, but not for the few copies of a short-lived context, whose
+// sum starts again with the next one; and no more than the array needs
 static void pinning()
 {
     hosthip::Stream s(0);
     std::vector<double> a(size_t(84) << 20), d(a.size());   // 704 MB
+    size_t slots = 0;
     auto passes = [&](size_t bytes, int n) {
         int pinned = 0;
+        slots = 0;
         nuctransfer::retain();
         for (int i = 0; i < n; i++) {
             nuctransfer::copy(d.data(), a.data(), bytes, hipMemcpyHostToDevice, &s);
             nuctransfer::copy(a.data(), d.data(), bytes, hipMemcpyDeviceToHost, &s);
             if (!pinned && !hosthip::pinned.empty()) pinned = i + 1;
+            slots = 0;
+            for (auto &p : hosthip::pinned) slots += p.second.bytes >> 22;
         }
         nuctransfer::release();
         CHECK(hosthip::pinned.empty(), "given back");
         return pinned;
     };
-    const size_t c96 = 40 * 96 * 96 * 96, c76 = 40 * 76 * 76 * 76;
+    const size_t c96 = 40 * 96 * 96 * 96, c76 = 40 * 76 * 76 * 76, c64 = 40 * 64 * 64 * 64;
     for (int contexts = 0; contexts < 6; contexts++) CHECK(passes(c96, 2) == 0, "96^3, two passes");
-    const int p96 = passes(c96, 12), p76 = passes(c76, 40);
-    CHECK(p96 >= 4 && p96 <= 6, "96^3: pass %d", p96);
-    CHECK(p76 >= 20 && p76 <= 40, "76^3: pass %d", p76);
-    CHECK(passes(8 * a.size(), 1) == 1, "704 MB");
+    const int p96 = passes(c96, 6);
+    CHECK(p96 == 3 && slots == 9, "96^3: pass %d, %zu slots", p96, slots);
+    const int p76 = passes(c76, 20);
+    CHECK(p76 >= 7 && p76 <= 12 && slots == 5, "76^3: pass %d, %zu slots", p76, slots);
+    const int p64 = passes(c64, 30);
+    CHECK(p64 >= 10 && p64 <= 15 && slots == 3, "64^3: pass %d, %zu slots", p64, slots);
+    CHECK(passes(8 * a.size(), 1) == 1 && slots == 16, "704 MB: %zu slots", slots);
 }
 
 // A copy behind a stream's earlier work: contexts and serving loops come and go
