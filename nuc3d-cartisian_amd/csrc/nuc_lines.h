@@ -290,7 +290,10 @@ __device__ __forceinline__ void w5_diff(T f2, T f3, T d1, T d2, T d3, T d4, T e1
 // values, where a row has 75 to 210.  Rows formed twice, with a quotient for each
 // indicator the second time, cost registers instead: 5 % on average, hccs78 twice
 // the time in some forms; this is 0.6 %, at most 3 (kernels of hccs and WENO7).
-template <int SCH> constexpr bool z_type() { return SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78; }
+template <int SCH> constexpr bool z_type()
+{
+    return SCH == WENO5Z || SCH == WENO7JS || SCH == HCCS || SCH == HCCS77 || SCH == HCCS78;
+}
 struct LineScale {
     int k = 0;   // of the wave, in the place of a double's exponent
     __device__ __forceinline__ double down() const { return __hiloint2double((1023 << 20) - k, 0); }
@@ -554,8 +557,9 @@ __device__ __forceinline__ void line_half(const T *Lw, int m0r, int mstep, const
         // other row reads.
         // Measured with the shorter indicators and reciprocals of the same rows, us
         // x/y/z: CRWENO5/LF 192^3 367/412/414 -> 361/400/385, 256^3 818/903/885 ->
-        // 825/851/836 (the x sweep, which applies the update, spills 6 registers), with AUSM 914/968/950 -> 862/914/890; hccs/LF 256^3
-        // 1220/1212/1184 -> 1133/1130/1118.
+        // 825/851/836 (the x sweep, which applies the update, spills 6 registers),
+        // with AUSM 914/968/950 -> 862/914/890; hccs/LF 256^3 1220/1212/1184 ->
+        // 1133/1130/1118.
         constexpr int RAD5 = 2;   // the 5-point stencil's window is win[O..]
         constexpr int O = RAD - RAD5;
         Chunk<R, TS, NL> ch;
